@@ -7,8 +7,8 @@
 //       P0 = (x, y, z, m)   pair coordinate (FP32 absolute or supercell-relative) and mass;
 //                           non-sources carry a sentinel position so the cull rejects them
 //       P1 = (vx, vy, vz, c)         c = fast magnetosonic bound sqrt((gamma P + B^2)/rho)
-//       P2 = (h, 1/h, gfac, rho)     gfac = kernel-gradient prefactor
-//       P3 = (pr, ph, bdr, psr)      pr = (P + B^2/2)/rho^2, ph = P/rho^2, bdr = 1/rho^2, psr = psi/rho^2
+//       P2 = (h, 1/h, gfac, ph)      gfac = kernel-gradient prefactor, ph = P/rho^2
+//       P3 = (pr, rho / 2, bdr, psr) pr = (P + B^2/2)/rho^2, bdr = 1/rho^2, psr = psi/rho^2
 //       P4 = (Bx, By, Bz, psi)       (MHD only)
 //   * supercell table: per-cell particle start (exclusive scan of the per-cell histogram).
 //
@@ -128,30 +128,30 @@ __device__ __forceinline__ float kshape(int kern, float q)
     return 0.0f;
 }
 
-// Gradient scalar s with grad_i W_ij = s r_ij (gfac includes sigma and the h powers).
-__device__ __forceinline__ float kgrad(int kern, float rr, float invR, float q, float gfac)
+// Gradient scalar s with grad_i W_ij = s r_ij (gfac includes sigma and the h powers), 0 at r = 0 for
+// the splines and beyond the support. The Wendland support test is a clamp of 1 - q/2 to [0, 1], free
+// as an output modifier of the fused multiply-add.
+__device__ __forceinline__ float kslope(int kern, float invR, float q, float gfac)
 {
 #pragma clang fp contract(off)
-    float s;
     if (kern == 2) {
-        const float t = fmaf(-0.5f, q, 1.0f);
-        s = gfac * ((t * t) * t);
-        s = q < 2.0f ? s : 0.0f;
-    } else if (kern == 0) {
+        const float t = __builtin_amdgcn_fmed3f(fmaf(-0.5f, q, 1.0f), 0.0f, 1.0f);
+        return gfac * ((t * t) * t);
+    }
+    float g;
+    if (kern == 0) {
         const float gi = q * fmaf(2.25f, q, -3.0f);
         const float t = 2.0f - q;
         const float go = -0.75f * (t * t);
-        const float g = q < 1.0f ? gi : (q < 2.0f ? go : 0.0f);
-        s = (gfac * g) * invR;
+        g = q < 1.0f ? gi : (q < 2.0f ? go : 0.0f);
     } else {
         const float a = 3.0f - q, b = 2.0f - q, c = 1.0f - q;
         const float a2 = a * a, b2 = b * b, c2 = c * c;
         const float a4 = a2 * a2, b4 = b2 * b2, c4 = c2 * c2;
-        const float g = q < 1.0f ? fmaf(-75.0f, c4, fmaf(30.0f, b4, -5.0f * a4))
-                                 : (q < 2.0f ? fmaf(30.0f, b4, -5.0f * a4) : (q < 3.0f ? -5.0f * a4 : 0.0f));
-        s = (gfac * g) * invR;
+        g = q < 1.0f ? fmaf(-75.0f, c4, fmaf(30.0f, b4, -5.0f * a4))
+                     : (q < 2.0f ? fmaf(30.0f, b4, -5.0f * a4) : (q < 3.0f ? -5.0f * a4 : 0.0f));
     }
-    return rr > 0.0f ? s : 0.0f;
+    return (gfac * g) * invR;
 }
 
 __device__ __forceinline__ float fast_rsq(float x) { return __builtin_amdgcn_rsqf(x); }

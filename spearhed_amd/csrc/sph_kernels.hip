@@ -758,6 +758,13 @@ __device__ __forceinline__ int compact_group(uint32_t msk, int sb, const LaneMap
     return m.inwave ? gtot : 0;
 }
 
+// Gradient factor of the smoothing kernel (kslope), the h powers and sigma included.
+__device__ __forceinline__ float grad_factor(int kern, float sig, float h)
+{
+#pragma clang fp contract(off)
+    return (kern == 2) ? -5.0f * sig / (h * h * h * h * h) : sig / (h * h * h * h);
+}
+
 // K partial sums of a target combined in lane order (deterministic); then one lane per particle
 // writes rho, the neighbour count and the interaction records of the force pass, and the run's
 // fast-speed maximum (cleaning speed) is raised.
@@ -784,7 +791,7 @@ __device__ __forceinline__ void density_finish(const RunDev& R, int r, StateBuf&
 #pragma clang fp contract(off)
         const float sig = R.sigma;
         const float wfac = sig / (h * h * h);
-        const float gfac = (kern == 2) ? -5.0f * sig / (h * h * h * h * h) : sig / (h * h * h * h);
+        const float gfac = grad_factor(kern, sig, h);
         float rho;
         if (tgt) {
             rho = wfac * (acc_t + m_own * R.f0);
@@ -802,8 +809,8 @@ __device__ __forceinline__ void density_finish(const RunDev& R, int r, StateBuf&
         const float psr = psi * bdr;
         const float c = sqrtf((gam * P + B2) * invrho);
         W.P1[i] = make_float4(vx, vy, vz, c);
-        W.P2[i] = make_float4(h, invh, gfac, rho);
-        W.P3[i] = make_float4(pr, ph, bdr, psr);
+        W.P2[i] = make_float4(h, invh, gfac, ph);
+        W.P3[i] = make_float4(pr, 0.5f * rho, bdr, psr);
         if (MHD) W.P4[i] = make_float4(bx, by, bz, psi);
         if (tgt) cmax = c;
     }
@@ -980,71 +987,88 @@ struct ForceAcc {
     float Ti, Tj, TBx, TBy, TBz, VBx, VBy, VBz, DB, PSx, PSy, PSz;
 };
 
-// ONE_H: every particle of the pair's run has the same smoothing length h; the pair then takes
-// s_j = s_i and the mean h = h without testing or forming them (the same bits: 0.5 (h + h) = h).
-template <bool MHD, bool ONE_H = false>
+// Per-run constants of the pair loop. alpha <= 0 switches the viscosity off with both coefficients 0, so
+// the loop has no branch for it (the term is then an exact zero).
+struct PairConst {
+    int kern;
+    float beta;               // of the signal speed
+    float va, vb;             // alpha / 2 and beta of the viscosity
+    float h, invh, gfac, e;   // ONE_H: the run's one smoothing length, 1/h, gradient factor and 0.01 h^2
+
+    __device__ __forceinline__ PairConst(const RunDev& R, int kern_, float h_, float gfac_)
+        : kern(kern_), beta(R.beta), va(R.alpha > 0.0f ? 0.5f * R.alpha : 0.0f), vb(R.alpha > 0.0f ? R.beta : 0.0f),
+          h(h_), invh(1.0f / h_), gfac(gfac_), e((0.01f * h_) * h_)
+    {
+    }
+};
+
+// The pair terms of target o and neighbour q, added to A. Records: 0 (x, y, z, m), 1 (v, c),
+// 2 (h, 1/h, gfac, ph), 3 (pr, rho / 2, bdr, psr), 4 (B, psi).
+// ONE_H: every particle of the run has the same smoothing length, so record 2 of the neighbour is not
+// read; the same bits as the general form. The pass is bound by VALU issue, so the pair is a straight
+// run of 72 instructions (three transcendental) with no branch or select in it: the support test is the
+// clamp of kslope, the r > 0 guard a lower bound on r2 (coincident particles then have r = 0, a finite
+// 1/r and exact zeros in every term), runs without viscosity or cleaning take zeros through the same
+// code, and the exact halves and doublings of the viscosity are folded away (rho / 2 in the record:
+// 1 / (rho_i/2 + rho_j/2) is the mean density's reciprocal). Every product and fused multiply-add is
+// written out, contraction off, so all instantiations round alike. Against the branched form with five
+// staged records (85 instructions) the force pass took 0.75 -> 0.69 ms at 2,097,152 particles.
+template <bool MHD, bool ONE_H>
 __device__ __forceinline__ void force_pair(const float4& o0, const float4& o1, const float4& o2, const float4& o3,
                                            const float4& o4, const float4& q0, const float4& q1, const float4& q2,
-                                           const float4& q3, const float4& q4, int kern, float alpha, float beta,
-                                           bool mhd, bool clean, ForceAcc& A)
+                                           const float4& q3, const float4& q4, const PairConst& C, ForceAcc& A)
 {
+#pragma clang fp contract(off)
     float dx, dy, dz;
     const float r2 = geom_r2(o0.x, o0.y, o0.z, q0, dx, dy, dz);
-    const float invR = r2 > 0.0f ? fast_rsq(r2) : 0.0f;
+    const float invR = fast_rsq(fmaxf(r2, 1e-37f));
     const float rr = r2 * invR;
-    const float s_i = kgrad(kern, rr, invR, rr * o2.y, o2.z);
-    // equal smoothing lengths (the records hold h, 1/h and the gradient factor derived from it)
-    // give the same gradient bit for bit: the second evaluation is skipped then
-    float s_j = s_i;
-    if (!ONE_H && __builtin_expect(q2.x != o2.x, 0)) s_j = kgrad(kern, rr, invR, rr * q2.y, q2.z);
+    const float ms_i = q0.w * kslope(C.kern, invR, rr * (ONE_H ? C.invh : o2.y), ONE_H ? C.gfac : o2.z);
+    float ms_j = ms_i;
+    // equal smoothing lengths give the same gradient bit for bit: the second evaluation is skipped then
+    if (!ONE_H && __builtin_expect(q2.x != o2.x, 0)) ms_j = q0.w * kslope(C.kern, invR, rr * q2.y, q2.z);
     const float dvx = o1.x - q1.x, dvy = o1.y - q1.y, dvz = o1.z - q1.z;
-    const float vr = dvx * dx + dvy * dy + dvz * dz;
-    const float m = q0.w;
-    const float ms_i = m * s_i, ms_j = m * s_j;
-    const float fiso = o3.x * ms_i + q3.x * ms_j;
-    A.ax -= fiso * dx;
-    A.ay -= fiso * dy;
-    A.az -= fiso * dz;
-    A.DV += ms_i * vr;
-    const float w = vr * invR;
-    const float vs = o1.w + q1.w - beta * fminf(w, 0.0f);
+    const float vr = fmaf(dvz, dz, fmaf(dvx, dx, dvy * dy));
+    const float fiso = fmaf(o3.x, ms_i, q3.x * ms_j);
+    A.ax = fmaf(-fiso, dx, A.ax);
+    A.ay = fmaf(-fiso, dy, A.ay);
+    A.az = fmaf(-fiso, dz, A.az);
+    A.DV = fmaf(ms_i, vr, A.DV);
+    const float vrm = fminf(vr, 0.0f);  // receding pairs: no viscosity
+    const float cs = o1.w + q1.w;
+    const float vs = fmaf(-C.beta, vrm * invR, cs);
     // signal speeds are >= +0, so their float bits order as integers: an integer max is the float
     // max without the NaN-quieting copy fmaxf needs for its loop-carried operand
     A.vmax = __int_as_float(max(__float_as_int(A.vmax), __float_as_int(vs)));
-    if (alpha > 0.0f) {  // uniform per run; receding pairs get mu = 0, hence Pi = 0
-        const float hb = ONE_H ? o2.x : 0.5f * (o2.x + q2.x);
-        const float mu = hb * fminf(vr, 0.0f) * fast_rcp(r2 + 0.01f * hb * hb);
-        // Pi = (beta mu - alpha cb) mu / rb, cb and rb the pair's mean sound speed and density, and
-        // gv = Pi (m s_i + m s_j) / 2. The halves are power-of-two scalings, exact in FP32: alpha cb
-        // = (alpha / 2)(c_i + c_j), and (1 / rb) / 2 = 1 / (rho_i + rho_j), so Ph = Pi / 2.
-        const float Ph = (beta * mu - (0.5f * alpha) * (o1.w + q1.w)) * mu * fast_rcp(o2.w + q2.w);
-        const float gv = Ph * (ms_i + ms_j);
-        A.ax -= gv * dx;
-        A.ay -= gv * dy;
-        A.az -= gv * dz;
-        A.AVU += gv * vr;
-    }
-    if (MHD && mhd) {
-        const float Bir = o4.x * dx + o4.y * dy + o4.z * dz;
-        const float Bjr = q4.x * dx + q4.y * dy + q4.z * dz;
-        const float ti = Bir * o3.z * ms_i;
-        const float tj = Bjr * q3.z * ms_j;
-        A.Ti += ti;
-        A.Tj += tj;
-        A.TBx += tj * q4.x;
-        A.TBy += tj * q4.y;
-        A.TBz += tj * q4.z;
+    // Pi = (beta mu - alpha cb) mu / rb, cb and rb the pair's mean sound speed and density, and
+    // gv = Pi (m s_i + m s_j) / 2
+    const float hb = ONE_H ? C.h : 0.5f * (o2.x + q2.x);
+    const float mu = (hb * vrm) * fast_rcp(r2 + (ONE_H ? C.e : (0.01f * hb) * hb));
+    const float Pi = (mu * fmaf(C.vb, mu, -(C.va * cs))) * fast_rcp(o3.y + q3.y);
+    const float gv = (ONE_H ? ms_i : 0.5f * (ms_i + ms_j)) * Pi;
+    A.ax = fmaf(-gv, dx, A.ax);
+    A.ay = fmaf(-gv, dy, A.ay);
+    A.az = fmaf(-gv, dz, A.az);
+    A.AVU = fmaf(gv, vr, A.AVU);
+    if constexpr (MHD) {
+        const float fps = fmaf(o3.w, ms_i, q3.w * ms_j);
+        A.PSx = fmaf(fps, dx, A.PSx);
+        A.PSy = fmaf(fps, dy, A.PSy);
+        A.PSz = fmaf(fps, dz, A.PSz);
+        const float Bir = fmaf(o4.z, dz, fmaf(o4.x, dx, o4.y * dy));
+        const float Bjr = fmaf(q4.z, dz, fmaf(q4.x, dx, q4.y * dy));
+        const float bj = Bjr * q3.z;
+        const float tj = bj * ms_j;
+        A.TBx = fmaf(tj, q4.x, A.TBx);
+        A.TBy = fmaf(tj, q4.y, A.TBy);
+        A.TBz = fmaf(tj, q4.z, A.TBz);
+        A.Ti = fmaf(Bir * o3.z, ms_i, A.Ti);
+        A.Tj = fmaf(bj, ms_j, A.Tj);
         const float wv = ms_i * Bir;
-        A.VBx += wv * dvx;
-        A.VBy += wv * dvy;
-        A.VBz += wv * dvz;
-        A.DB += ms_i * (Bir - Bjr);
-        if (clean) {
-            const float fps = o3.w * ms_i + q3.w * ms_j;
-            A.PSx += fps * dx;
-            A.PSy += fps * dy;
-            A.PSz += fps * dz;
-        }
+        A.VBx = fmaf(wv, dvx, A.VBx);
+        A.VBy = fmaf(wv, dvy, A.VBy);
+        A.VBz = fmaf(wv, dvz, A.VBz);
+        A.DB = fmaf(ms_i, Bir - Bjr, A.DB);
     }
 }
 
@@ -1054,7 +1078,7 @@ __device__ __forceinline__ void force_write(const RunDev& R, WorkBuf& W, const F
                                             const float4& o2, const float4& o3, const float4& o4, bool mhd,
                                             bool clean, float borve, float ch)
 {
-    const float rho = o2.w;
+    const float rho = 2.0f * o3.y;
     const float invrho = 1.0f / rho;
     float ax = T.ax, ay = T.ay, az = T.az;
     if (MHD && mhd) {
@@ -1066,7 +1090,7 @@ __device__ __forceinline__ void force_write(const RunDev& R, WorkBuf& W, const F
     W.dvdt[0][i] = ax;
     W.dvdt[1][i] = ay;
     W.dvdt[2][i] = az;
-    W.dudt[i] = o3.y * T.DV + 0.5f * T.AVU;
+    W.dudt[i] = o2.w * T.DV + 0.5f * T.AVU;
     W.vsig[i] = fmaxf(2.0f * o1.w, T.vmax);
     if (MHD && mhd) {
         const float divB = -T.DB * invrho;
@@ -1177,10 +1201,15 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
     if (writer && tgt) force_write<MHD>(R, W, T, i, o1, o2, o3, o4, mhd, clean, borve, ch);
 }
 
+// Records staged per neighbour: P0, P1, P3, P4 with MHD fields, and P2 unless the run has one smoothing
+// length (64 instead of 80 bytes per neighbour).
+template <bool MHD, bool ONE_H>
+constexpr int kForcePlanes = 3 + (MHD ? 1 : 0) + (ONE_H ? 0 : 1);
+
 template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX, bool ONE_H = false>
 __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ runs, int nruns, int ncell_tot,
                                             int nblk_total, StateBuf& S, WorkBuf& W, int kmax, NbListR<RMAX>& L,
-                                            float4 (&sp)[MHD ? 5 : 4][CH], ListT<CH> (&lst)[BAL == 1 ? 64 * 32 : 1],
+                                            float4 (&sp)[kForcePlanes<MHD, ONE_H>][CH], ListT<CH> (&lst)[BAL == 1 ? 64 * 32 : 1],
                                             PreList& P)
 {
     constexpr int NS = RMAX == 1 ? 27 : 125;
@@ -1229,7 +1258,8 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
     const int chk = per * K;
     const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
     const float H2 = R.H2;
-    const float alpha = R.alpha, beta = R.beta;
+    const float h_own = S.h[t0];  // the run's one smoothing length (ONE_H)
+    const PairConst pc(R, kern, h_own, grad_factor(kern, R.sigma, h_own));
     const bool mhd = MHD && R.mhd;
     const bool clean = mhd && R.cleaning;
     const float borve = mhd ? R.borve : 0.0f;
@@ -1243,7 +1273,9 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
         const bool valid = lm.inwave && t < nt;
         const int i = t0 + (valid ? t : 0);
         const bool tgt = valid && is_target(S.species[i], S.mask[i]);
-        const float4 o0 = W.P0[i], o1 = W.P1[i], o2 = W.P2[i], o3 = W.P3[i];
+        const float4 o0 = W.P0[i], o1 = W.P1[i], o3 = W.P3[i];
+        float4 o2 = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (!ONE_H) o2 = W.P2[i];
         float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
         if (MHD) o4 = W.P4[i];
         // the self slot is needed only where the pass culls (a stored list implies stored masks)
@@ -1263,9 +1295,9 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
                     p.z += L.sh[sg][2];
                     sp[0][e] = p;
                     sp[1][e] = W.P1[j];
-                    sp[2][e] = W.P2[j];
-                    sp[3][e] = W.P3[j];
-                    if constexpr (MHD) sp[4][e] = W.P4[j];
+                    sp[2][e] = W.P3[j];
+                    if constexpr (MHD) sp[3][e] = W.P4[j];
+                    if constexpr (!ONE_H) sp[MHD ? 4 : 3][e] = W.P2[j];
                 } else {
                     sp[0][e] = make_float4(kSentinel, kSentinel, kSentinel, 0.0f);
                 }
@@ -1293,15 +1325,14 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
                         const int ii = __builtin_ctz(msk);
                         msk &= msk - 1;
                         const int eb = (int)__umul24((unsigned)ii, (unsigned)kb) + eb0;
-                        float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if constexpr (MHD) q4 = lds_at(sp[4], eb);
                         // all of the pair's records read before any is used: one LDS wait per pair
                         // instead of one per record (force pass 3% faster; same arithmetic)
-                        const float4 q0 = lds_at(sp[0], eb), q1 = lds_at(sp[1], eb), q2 = lds_at(sp[2], eb),
-                                     q3 = lds_at(sp[3], eb);
+                        const float4 q0 = lds_at(sp[0], eb), q1 = lds_at(sp[1], eb), q3 = lds_at(sp[2], eb);
+                        float4 q2 = make_float4(0.f, 0.f, 0.f, 0.f), q4 = q2;
+                        if constexpr (MHD) q4 = lds_at(sp[3], eb);
+                        if constexpr (!ONE_H) q2 = lds_at(sp[MHD ? 4 : 3], eb);
                         __builtin_amdgcn_sched_barrier(0);
-                        force_pair<MHD, ONE_H>(o0, o1, o2, o3, o4, q0, q1, q2, q3, q4, kern, alpha, beta, mhd, clean,
-                                               A);
+                        force_pair<MHD, ONE_H>(o0, o1, o2, o3, o4, q0, q1, q2, q3, q4, pc, A);
                     }
                 } else {
                     const int gtot = compact_group(msk, sb, lm, lst);
@@ -1309,19 +1340,19 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
                     const ListT<CH>* mine = lst + lm.gfirst * 32;  // this target's accepted slots
                     for (int q = k; q < gtot; q += K) {
                         const int eb = (int)sizeof(float4) * (int)mine[q];
-                        float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if constexpr (MHD) q4 = lds_at(sp[4], eb);
-                        const float4 q0 = lds_at(sp[0], eb), q1 = lds_at(sp[1], eb), q2 = lds_at(sp[2], eb),
-                                     q3 = lds_at(sp[3], eb);
+                        const float4 q0 = lds_at(sp[0], eb), q1 = lds_at(sp[1], eb), q3 = lds_at(sp[2], eb);
+                        float4 q2 = make_float4(0.f, 0.f, 0.f, 0.f), q4 = q2;
+                        if constexpr (MHD) q4 = lds_at(sp[3], eb);
+                        if constexpr (!ONE_H) q2 = lds_at(sp[MHD ? 4 : 3], eb);
                         __builtin_amdgcn_sched_barrier(0);
-                        force_pair<MHD, ONE_H>(o0, o1, o2, o3, o4, q0, q1, q2, q3, q4, kern, alpha, beta, mhd, clean,
-                                               A);
+                        force_pair<MHD, ONE_H>(o0, o1, o2, o3, o4, q0, q1, q2, q3, q4, pc, A);
                     }
                     __syncthreads();
                 }
             }
             __syncthreads();
         }
+        if constexpr (ONE_H) o2 = W.P2[i];
         force_finish<MHD>(R, W, lm, A, tgt, i, o1, o2, o3, o4, mhd, clean, borve, ch);
     }
 }
@@ -1333,9 +1364,8 @@ __attribute__((amdgpu_waves_per_eu(BAL == 1 && !GRID ? 5 : 1)))
 void k_forces(const RunDev* __restrict__ runs, int nruns, int ncell_tot, int nblk_total, StateBuf S, WorkBuf W,
               int kmax, int balance)
 {
-    constexpr int NP = MHD ? 5 : 4;
     __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[NP][CH];
+    __shared__ float4 sp[kForcePlanes<MHD, ONE_H && !GRID>][CH];
     __shared__ ListT<CH> lst[BAL == 1 ? 64 * 32 : 1];  // compaction lists of the balanced pair loop
     __shared__ PreList P;
     if constexpr (GRID) {
@@ -1507,7 +1537,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
     const bool keep = nt <= lm.tpg && Lr <= 32 * kMaskWords;  // the density pass stored masks
     const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
     const float H2 = R.H2;
-    const float alpha = R.alpha, beta = R.beta;
+    const PairConst pc(R, kern, 1.0f, 0.0f);
     const bool mhd = MHD && R.mhd;
     const bool clean = mhd && R.cleaning;
     const float borve = mhd ? R.borve : 0.0f;
@@ -1579,8 +1609,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
                     const int e = (int)lst[lo + q] - base;
                     float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
                     if constexpr (MHD) q4 = sp[4][e];
-                    force_pair<MHD>(o0, o1, o2, o3, o4, sp[0][e], sp[1][e], sp[2][e], sp[3][e], q4, kern, alpha,
-                                    beta, mhd, clean, A);
+                    force_pair<MHD, false>(o0, o1, o2, o3, o4, sp[0][e], sp[1][e], sp[2][e], sp[3][e], q4, pc, A);
                 }
                 lo += g;
             } else {
@@ -1602,8 +1631,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
                         const int e = cc - base + ii;
                         float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
                         if constexpr (MHD) q4 = sp[4][e];
-                        force_pair<MHD>(o0, o1, o2, o3, o4, sp[0][e], sp[1][e], sp[2][e], sp[3][e], q4, kern, alpha,
-                                        beta, mhd, clean, A);
+                        force_pair<MHD, false>(o0, o1, o2, o3, o4, sp[0][e], sp[1][e], sp[2][e], sp[3][e], q4, pc, A);
                     }
                 }
             }
