@@ -138,7 +138,8 @@ typedef struct sph_grid_info {
 
 /* Launch tunables chosen by the autotuner (sph_autotune). */
 typedef struct sph_tuning {
-    int32_t density_chunk;  /* neighbour candidates staged in LDS per chunk by the density pass: 128|256|512 */
+    int32_t density_chunk;  /* density pass: 128 and 256 are taken alike (256 LDS slots per wave, 160 candidates
+                               per chunk beside the kept list); 512: the whole-supercell pass */
     int32_t force_chunk;    /* neighbour records staged in LDS per chunk by the force pass: 64|128 */
     int32_t waves_per_cu;   /* pair passes: 0 = one wave per supercell (default); 1..64 = a persistent
                                grid of waves_per_cu x (compute units) waves, each walking the supercells

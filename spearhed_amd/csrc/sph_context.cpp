@@ -104,12 +104,6 @@ int fail(sph_ctx* c, int code, const std::string& msg)
 
 int support_of(int kernel) { return kernel == SPH_KERNEL_QUINTIC ? 3 : 2; }
 
-float f0_of(int kernel)
-{
-    if (kernel == SPH_KERNEL_QUINTIC) return 66.0f;  // 3^5 - 6*2^5 + 15
-    return 1.0f;
-}
-
 float sigma_of(int kernel)
 {
     const float pi = 3.14159265358979323846f;
@@ -139,8 +133,7 @@ bool make_run(const sph_run_config& c, RunDev& R, std::string& why)
     }
     if (std::isnan(c.dt_fixed) || std::isinf(c.dt_fixed)) { why = "dt_fixed must be finite"; return false; }
     if (std::isnan(c.cell_factor) || std::isinf(c.cell_factor)) { why = "cell_factor must be finite"; return false; }
-    R.support = support_of(c.kernel);
-    R.H = (float)R.support * c.h0;
+    R.H = (float)support_of(c.kernel) * c.h0;
     R.H2 = R.H * R.H;
     const double f = cell_factor_of(c.cell_factor);
     R.reach = f < 1.0 ? 2 : 1;
@@ -160,7 +153,7 @@ bool make_run(const sph_run_config& c, RunDev& R, std::string& why)
         int n = (int)nd;
         if (n < 1) n = 1;
         R.n[a] = n;
-        R.periodic[a] = c.periodic[a] ? 1 : 0;
+        if (c.periodic[a]) R.flags |= 1u << a;
         R.lo[a] = c.box_lo[a];
         R.L[a] = L;
         R.s[a] = L / (double)n;
@@ -173,9 +166,10 @@ bool make_run(const sph_run_config& c, RunDev& R, std::string& why)
     }
     if (nc > (1LL << 30)) { why = "too many supercells"; return false; }
     R.ncell = (int32_t)nc;
-    R.kernel = c.kernel;
-    R.mhd = c.mhd ? 1 : 0;
-    R.cleaning = (c.mhd && c.cleaning) ? 1 : 0;
+    for (int a = 0; a < 2; ++a) R.div[a] = div_multiplier((uint32_t)R.n[a]);
+    if (c.mhd) R.flags |= 1u << 3;
+    if (c.mhd && c.cleaning) R.flags |= 1u << 4;
+    R.flags |= (uint32_t)c.kernel << 8;
     R.gamma = c.gamma;
     R.alpha = c.alpha_visc;
     R.beta = c.beta_visc;
@@ -184,7 +178,12 @@ bool make_run(const sph_run_config& c, RunDev& R, std::string& why)
     R.cfl = c.cfl;
     R.cfl_force = c.cfl_force;
     R.sigma = sigma_of(c.kernel);
-    R.f0 = f0_of(c.kernel);
+    // the factors of one particle's density and gradient, in the device's own FP32 operations and order
+    const float h = c.h0;
+    R.h0 = h;
+    R.inv_h0 = 1.0f / h;
+    R.wfac0 = R.sigma / (h * h * h);
+    R.gfac0 = c.kernel == SPH_KERNEL_WENDLAND ? -5.0f * R.sigma / (h * h * h * h * h) : R.sigma / (h * h * h * h);
     R.dt_fixed = c.dt_fixed;
     return true;
 }
@@ -1456,10 +1455,9 @@ int sph_autotune(sph_ctx* c, int32_t n_steps, sph_tuning* best)
     // supercell edges of 1 and 1.15 interaction radii, one wave per supercell; then the winner's
     // persistent-grid variants (waves per compute unit)
     std::vector<sph_tuning> cands;
-    for (int dc : {128, 256})
-        for (int fc : {64, 128})
-            for (int k : {16, 64})
-                for (int bal : {0, 1}) cands.push_back({dc, fc, 0, k, bal});
+    for (int fc : {64, 128})
+        for (int k : {16, 64})
+            for (int bal : {0, 1}) cands.push_back({128, fc, 0, k, bal});
     for (int k : {16, 64}) cands.push_back({512, 128, 0, k, 2});
     // supercell edges of 1/2, 1 and 1.15 interaction radii, each no finer than the run's own setting;
     // a grid the context's supercell table cannot hold is skipped (a context reserves cells for its

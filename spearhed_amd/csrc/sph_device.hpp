@@ -27,17 +27,38 @@ struct RunDev {
     int64_t p0, np;          // first particle, particle count
     int32_t c0, ncell;       // first supercell, supercell count
     int32_t n[3];            // supercells per axis
-    int32_t periodic[3];
+    uint32_t flags;          // bits 0..2: periodic axes; 3: MHD; 4: cleaning; 8..9: smoothing kernel
+    uint32_t div[2];         // multipliers of the division by n[0] and n[1] (div_by), on the scalar unit
     double lo[3], L[3], s[3], inv_s[3];
     float lo32[3], L32[3], s32[3], inv_s32[3];
     float H, H2;             // interaction radius and its square (FP32, as used by the cull)
-    int32_t kernel, mhd, cleaning, support;
     float gamma, alpha, beta, borve, clean_sigma, cfl, cfl_force, sigma;
     double dt_fixed;
     int32_t kb_first, kb_count;  // particle-kernel blocks of this run
-    float f0;                    // kernel shape at q = 0
+    float h0, inv_h0, wfac0, gfac0;  // the configured smoothing length, 1/h0 and the density and gradient factors
+                                     // of it: waves whose targets all have it divide nothing
     int32_t reach;               // supercells the stencil reaches per side: 1 (edge >= H) or 2 (edge >= H/2)
 };
+
+static_assert(sizeof(RunDev) == 272, "the pool's reservation counts it");
+
+// fields of RunDev::flags
+__device__ __forceinline__ bool run_periodic(uint32_t flags, int a) { return (flags >> a) & 1u; }
+__device__ __forceinline__ bool run_mhd(uint32_t flags) { return (flags >> 3) & 1u; }
+__device__ __forceinline__ bool run_cleaning(uint32_t flags) { return (flags >> 4) & 1u; }
+__device__ __forceinline__ int run_kernel(uint32_t flags) { return (int)((flags >> 8) & 3u); }
+
+// x / n for 0 <= x < 2^31 with the multiplier floor(2^(31 + s) / n) + 1, s = ceil(log2 n): the excess of
+// multiplier * n over 2^(31 + s) is at most n <= 2^s, so x times it never reaches the next quotient.
+__host__ __device__ __forceinline__ uint32_t div_shift(uint32_t n) { return 32u - (uint32_t)__builtin_clz(n - 1u); }
+__host__ inline uint32_t div_multiplier(uint32_t n)
+{
+    return n < 2 ? 0u : (uint32_t)((uint64_t(1) << (31 + div_shift(n))) / n) + 1u;
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t x, uint32_t n, uint32_t mul)
+{
+    return n < 2 ? x : __umulhi(x, mul) >> (div_shift(n) - 1u);
+}
 
 // Device arrays of one particle buffer set.
 struct StateBuf {
@@ -107,8 +128,9 @@ __device__ __forceinline__ float kshape(int kern, float q)
 {
 #pragma clang fp contract(off)
     if (kern == 2) {  // Wendland C2: (1 - q/2)^4 (1 + 2q)
-        // 1 - q/2 clamped at 0: exactly 0 for q >= 2 (the support test), the same bits below it
-        const float t = fmaxf(fmaf(-0.5f, q, 1.0f), 0.0f);
+        // 1 - q/2 clamped to [0, 1]: exactly 0 for q >= 2 (the support test), the same bits below it; the
+        // clamp is an output modifier of the fused multiply-add
+        const float t = __builtin_amdgcn_fmed3f(fmaf(-0.5f, q, 1.0f), 0.0f, 1.0f);
         const float t2 = t * t;
         return (t2 * t2) * fmaf(2.0f, q, 1.0f);
     }
@@ -127,6 +149,9 @@ __device__ __forceinline__ float kshape(int kern, float q)
     if (q < 3.0f) return a5;
     return 0.0f;
 }
+
+// f(0): 3^5 - 6 2^5 + 15 of the quintic, 1 of the others.
+__device__ __forceinline__ float kshape0(int kern) { return kern == 1 ? 66.0f : 1.0f; }
 
 // Gradient scalar s with grad_i W_ij = s r_ij (gfac includes sigma and the h powers), 0 at r = 0 for
 // the splines and beyond the support. The Wendland support test is a clamp of 1 - q/2 to [0, 1], free

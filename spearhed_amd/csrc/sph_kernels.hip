@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ ru
                 double x = S.pos64[a][i];
                 if (mov) {
                     x = x + (double)S.vel[a][i] * dt;
-                    if (R.periodic[a]) {
+                    if (run_periodic(R.flags, a)) {
                         double hi = R.lo[a] + R.L[a];
                         if (x >= hi) x = x - R.L[a];
                         else if (x < R.lo[a]) x = x + R.L[a];
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ ru
                 float x = S.pos32[a][i];
                 if (mov) {
                     x = x + S.vel[a][i] * (float)dt;
-                    if (R.periodic[a]) {
+                    if (run_periodic(R.flags, a)) {
                         float hi = R.lo32[a] + R.L32[a];
                         if (x >= hi) x = x - R.L32[a];
                         else if (x < R.lo32[a]) x = x + R.L32[a];
@@ -319,9 +319,10 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
 // ------------------------------------------------------------------------------------------------
 template <int NS>
 struct NbListT {
-    int start[NS];
-    int off[NS + 1];  // entries past the run's stencil hold the total, so no search selects them
-    float sh[NS][3];
+    float4 t[NS];     // staged-position shift of a stencil supercell (x, y, z) and its first particle less its first
+                      // list index (int bits): list index v of that supercell is particle v + this
+    int off[NS + 1];  // list index of its first candidate; entries past the run's stencil hold the total, so no
+                      // search selects them
 };
 template <int RMAX>
 using NbListR = NbListT<RMAX == 1 ? 27 : 125>;
@@ -329,18 +330,105 @@ using NbListR = NbListT<RMAX == 1 ? 27 : 125>;
 template <int CH>
 using ListT = typename std::conditional<(CH <= 256), uint8_t, uint16_t>::type;
 
+// Arguments of the pair passes. The kernels read them where they are used, from the kernel-argument
+// segment (the struct is their only parameter, at its start): as plain parameters some fifty pointers are
+// loaded at the entry, more than the scalar registers hold, and the spills cost vector instructions
+// (350 of a density wave's 2,500).
+struct PairArgs {
+    const RunDev* runs;
+    int nruns, ncell_tot, nblk_total, kmax;
+    StateBuf S;
+    WorkBuf W;
+};
+__device__ __forceinline__ const PairArgs& pair_args()
+{
+    return *(const PairArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// A run's constants in the constant address space: scalar loads wherever they are used, also after the
+// wave's own stores (no pair pass writes the table).
+using RunC = const __attribute__((address_space(4))) RunDev;
+
+// A value that is the same in every lane, moved to a scalar register: what follows from it is then
+// computed by the scalar unit instead of taking vector issue slots (the pair passes are bound by them).
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// x / d for uniform x, d > 0 (1 / d given to within an ulp or two): the float quotient of x + 1/2 stays at
+// least 1/(2 d) away from the next whole number, more than its rounding error below 2^20; larger x divide.
+__device__ __forceinline__ int quot(int x, int d, float rd)
+{
+    return x < (1 << 20) ? (int)(((float)x + 0.5f) * rd) : x / d;
+}
+__device__ __forceinline__ int uquot(int x, int d, float rd) { return uniform(quot(x, d, rd)); }
+
+// Element at a 32-bit byte offset from a uniform base: the offset is one vector register and the base
+// stays in scalar ones (no 64-bit vector address arithmetic). A context holds at most 2^30 particles, so
+// columns of up to four bytes are reached from their start; 16-byte records from the wave's first one.
+template <class T>
+__device__ __forceinline__ T& at32(T* base, uint32_t byte_off)
+{
+    return *(T*)((char*)base + byte_off);
+}
+
+// Particle t (per lane) of the supercell whose first particle is t0 (uniform): offsets of its columns.
+struct Slot {
+    int t0;
+    uint32_t i;    // index in a column
+    uint32_t t16;  // byte offset of its record from that of t0
+
+    __device__ __forceinline__ Slot(int t0_, uint32_t t) : t0(t0_), i((uint32_t)t0_ + t), t16(t * 16u) {}
+    template <class T>
+    __device__ __forceinline__ T& col(T* base) const
+    {
+        static_assert(sizeof(T) <= 4, "a wider column needs a 64-bit offset");
+        return at32(base, i * (uint32_t)sizeof(T));
+    }
+    __device__ __forceinline__ float4& rec(float4* base) const { return at32(base + t0, t16); }
+};
+
+// Inclusive sum over the lanes of a wave by DPP row shifts and row broadcasts (six additions).
+__device__ __forceinline__ int dpp_incl_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
+// Maximum over the wave of values whose bits order as unsigned integers (floats >= +0), as a uniform.
+__device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, false);
+        v = v > o ? v : o;
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Neighbour supercell `seg` of cell c in a stencil of side 2 reach + 1 (x fastest, offsets
 // d = seg % side - reach, ...): returns false outside a non-periodic axis; else the global cell and
 // the staged-position shift (the periodic image for FP32 absolute coordinates, d * cell edge for
 // supercell-relative ones). A 1-cell periodic axis is wrapped twice by a reach of 2.
 template <bool MIXED, int RMAX>
-__device__ __forceinline__ bool nb_cell(const RunDev& R, const int c[3], int seg, int& cc, float sh[3])
+__device__ __forceinline__ bool nb_cell(RunC& R, const int c[3], int seg, int& cc, float sh[3])
 {
     int d[3];
-    if (RMAX == 1) {
-        d[0] = seg % 3 - 1;
-        d[1] = (seg / 3) % 3 - 1;
-        d[2] = seg / 9 - 1;
+    if (RMAX == 1) {  // seg < 64: quotients by 9 and 3 as multiply-shifts
+        const int z = (int)(__umul24((unsigned)seg, 57u) >> 9), yx = seg - 9 * z;
+        const int y = (int)(__umul24((unsigned)yx, 11u) >> 5);
+        d[0] = yx - 3 * y - 1;
+        d[1] = y - 1;
+        d[2] = z - 1;
     } else {
         const int r = R.reach, side = 2 * R.reach + 1;
         d[0] = seg % side - r;
@@ -352,7 +440,7 @@ __device__ __forceinline__ bool nb_cell(const RunDev& R, const int c[3], int seg
     for (int a = 0; a < 3; ++a) {
         int x = c[a] + d[a];
         int wrap = 0;
-        if (R.periodic[a]) {
+        if (run_periodic(R.flags, a)) {
             if (RMAX == 1) wrap = x < 0 ? -1 : (x >= R.n[a] ? 1 : 0);
             else wrap = x >= 0 ? x / R.n[a] : -((R.n[a] - 1 - x) / R.n[a]);
             x -= wrap * R.n[a];
@@ -368,22 +456,25 @@ __device__ __forceinline__ bool nb_cell(const RunDev& R, const int c[3], int seg
 
 // Index of the cell's own supercell in its stencil (the centre).
 template <int RMAX>
-__device__ __forceinline__ int self_segment(const RunDev& R)
+__device__ __forceinline__ int self_segment(RunC& R)
 {
     if (RMAX == 1) return 13;
     const int side = 2 * R.reach + 1;
     return (side * side * side - 1) / 2;
 }
 
+// Builds the list in LDS; returns its total and sets the list index of the cell's own first particle.
 template <bool MIXED, int RMAX>
-__device__ __forceinline__ void build_nblist(const RunDev& R, int lcell, const uint32_t* __restrict__ cs,
-                                             NbListR<RMAX>& L)
+__device__ __forceinline__ int build_nblist(RunC& R, int lcell, const uint32_t* __restrict__ cs,
+                                            NbListR<RMAX>& L, int& self_v0)
 {
     constexpr int NS = RMAX == 1 ? 27 : 125;
     const int lane = threadIdx.x;
-    const int c[3] = {lcell % R.n[0], (lcell / R.n[0]) % R.n[1], lcell / (R.n[0] * R.n[1])};
+    const uint32_t row = div_by((uint32_t)lcell, (uint32_t)R.n[0], R.div[0]);
+    const uint32_t plane = div_by(row, (uint32_t)R.n[1], R.div[1]);
+    const int c[3] = {lcell - (int)row * R.n[0], (int)row - (int)plane * R.n[1], (int)plane};
     const int side = RMAX == 1 ? 3 : 2 * R.reach + 1;
-    const int nseg = side * side * side;
+    const int nseg = RMAX == 1 ? 27 : side * side * side;
     int carry = 0;
 #pragma unroll
     for (int base = 0; base < NS; base += 64) {
@@ -397,19 +488,19 @@ __device__ __forceinline__ void build_nblist(const RunDev& R, int lcell, const u
                 cnt = (int)cs[cc + 1] - st;
             }
         }
-        const int incl = wave_incl_scan(cnt) + carry;
+        const int incl = dpp_incl_scan(cnt) + carry;
         if (seg < NS) {
-            L.start[seg] = st;
+            L.t[seg] = make_float4(sh[0], sh[1], sh[2], __int_as_float(st - (incl - cnt)));
             L.off[seg] = seg < nseg ? incl - cnt : 0;  // past the stencil: overwritten with the total below
-            L.sh[seg][0] = sh[0];
-            L.sh[seg][1] = sh[1];
-            L.sh[seg][2] = sh[2];
         }
-        carry = __shfl(incl, 63, 64);
+        if (RMAX == 1) self_v0 = __builtin_amdgcn_readlane(incl - cnt, 13);
+        carry = __builtin_amdgcn_readlane(incl, 63);
     }
     // the total after the last stencil entry, and in every entry past the run's stencil
     for (int k = nseg + lane; k <= NS; k += 64) L.off[k] = carry;
     __syncthreads();
+    if (RMAX != 1) self_v0 = uniform(L.off[self_segment<RMAX>(R)]);
+    return carry;
 }
 
 // segment of virtual index v (largest k with off[k] <= v, over non-decreasing off[0..NS-1])
@@ -433,53 +524,42 @@ __device__ __forceinline__ int nb_segment(const NbListT<NS>& L, int v)
 // before. With supercells of edge ~H about half of the 27-cell stencil goes (MHD turbulence at 2M
 // particles: 381 -> 194 candidates per supercell in a CPU replay), which halves the cull and the
 // staging and leaves fewer, fuller chunks for the pair loops. The density pass filters; the force
-// pass reads the kept list back from the mask row (recomputing it only where it was not stored),
-// 11% faster than with no filter; the density pass, bound by latency more than by its cull, is 3%
-// slower.
+// pass reads the kept list back from the mask row (recomputing it only where it was not stored).
 // ------------------------------------------------------------------------------------------------
 constexpr int kPreCap = 768;  // larger stencils, and supercells of more than 64 particles, stage whole
 
 struct PreList {
-    uint16_t v[kPreCap];  // the kept candidates in list order: list index, and for the 27-cell stencil
-                          // the segment in bits 10..14 (so staging needs no search)
+    union {
+        uint16_t v[kPreCap];       // the kept candidates in list order (pre_entry)
+        uint32_t v2[kPreCap / 2];  // the same, two entries per word
+    };
     uint16_t self_s[64];  // kept index of each target of the supercell (a target is always kept)
+    uint32_t seg4[64];    // see fill_segments
 };
 
-// A kept-list entry: the list index (< kPreCap <= 1024) and, for the 27-cell stencil, its segment.
+// A kept-list entry: the list index (< kPreCap <= 1024) and, for the 27-cell stencil, its segment, so that
+// staging needs no search.
 template <int NS>
 __device__ __forceinline__ uint16_t pre_entry(int v, int sg)
 {
     return (uint16_t)(NS == 27 ? v | (sg << 10) : v);
 }
 
-// List index and stencil segment of staged candidate su: from the kept list when the filter is on
-// (the segment packed in the entry for the 27-cell stencil, else searched), else su itself.
+// Particle index and position shift of list index v.
 template <int NS>
-__device__ __forceinline__ void staged_candidate(const NbListT<NS>& L, const PreList& P, bool pre, int su, int& v,
-                                                 int& sg)
+__device__ __forceinline__ int list_candidate(const NbListT<NS>& L, int v, float4& t)
 {
-    if (pre) {
-        const int e = P.v[su];
-        v = NS == 27 ? (e & 1023) : e;
-        sg = NS == 27 ? (e >> 10) : nb_segment(L, v);
-    } else {
-        v = su;
-        sg = nb_segment(L, v);
-    }
+    t = L.t[nb_segment(L, v)];
+    return v + __float_as_int(t.w);
 }
 
-__device__ __forceinline__ float wave_min(float x)
+// Particle index and position shift of the kept-list entry e.
+template <int NS>
+__device__ __forceinline__ int kept_candidate(const NbListT<NS>& L, int e, float4& t)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) x = fminf(x, __shfl_xor(x, off, 64));
-    return x;
-}
-
-__device__ __forceinline__ float wave_max(float x)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));
-    return x;
+    if (NS != 27) return list_candidate(L, e, t);
+    t = L.t[e >> 10];
+    return (e & 1023) + __float_as_int(t.w);
 }
 
 // Bounding box of the targets among a supercell's nt <= 64 particles (from their position records;
@@ -496,79 +576,153 @@ struct TargetBoxInput {
 
 __device__ __forceinline__ TargetBoxInput target_box_load(const StateBuf& S, const WorkBuf& W, int t0, int nt)
 {
-    const int lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x;
     TargetBoxInput in;
-    if (lane < nt) {
-        const int i = t0 + lane;
-        in.species = S.species[i];
-        in.mask = S.mask[i];
-        in.o = W.P0[i];  // a target is a source: its record holds its position
+    if ((int)lane < nt) {
+        in.species = at32(S.species + t0, lane);
+        in.mask = at32(S.mask + t0, lane);
+        in.o = at32(W.P0 + t0, lane * 16u);  // a target is a source: its record holds its position
     }
     return in;
+}
+
+// Minimum or maximum over a wave whose lanes past nt hold the neutral value: rotations within the
+// 16-lane rows (every lane reads a valid one, so each is one instruction), then the rows in use.
+template <bool MAX>
+__device__ __forceinline__ float wave_extreme(float x, int nt)
+{
+    auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : fminf(a, b); };
+    auto ror = [&](auto n) {
+        return __int_as_float(
+            __builtin_amdgcn_mov_dpp(__float_as_int(x), 0x120 + decltype(n)::value, 0xf, 0xf, true));
+    };
+    x = op(x, ror(std::integral_constant<int, 8>{}));
+    x = op(x, ror(std::integral_constant<int, 4>{}));
+    x = op(x, ror(std::integral_constant<int, 2>{}));
+    x = op(x, ror(std::integral_constant<int, 1>{}));
+    auto row = [&](int r) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 16 * r)); };
+    float m = row(0);
+    if (nt > 16) m = op(m, row(1));
+    if (nt > 32) m = op(op(m, row(2)), row(3));
+    return m;
 }
 
 __device__ __forceinline__ TargetBox target_box(const TargetBoxInput& in, int nt)
 {
     const bool has = (int)threadIdx.x < nt && is_target(in.species, in.mask);
     TargetBox b;
-    b.lx = wave_min(has ? in.o.x : INFINITY);
-    b.hx = wave_max(has ? in.o.x : -INFINITY);
-    b.ly = wave_min(has ? in.o.y : INFINITY);
-    b.hy = wave_max(has ? in.o.y : -INFINITY);
-    b.lz = wave_min(has ? in.o.z : INFINITY);
-    b.hz = wave_max(has ? in.o.z : -INFINITY);
+    b.lx = wave_extreme<false>(has ? in.o.x : INFINITY, nt);
+    b.hx = wave_extreme<true>(has ? in.o.x : -INFINITY, nt);
+    b.ly = wave_extreme<false>(has ? in.o.y : INFINITY, nt);
+    b.hy = wave_extreme<true>(has ? in.o.y : -INFINITY, nt);
+    b.lz = wave_extreme<false>(has ? in.o.z : INFINITY, nt);
+    b.hz = wave_extreme<true>(has ? in.o.z : -INFINITY, nt);
     return b;
 }
 
-// Keeps in P the candidates of the supercell's list (of `total`) that lie within the support radius
-// of its targets' bounding box B, and returns how many there are; with the filter off (`on` false)
-// returns `total` and leaves P unused.
+// Stencil segments of the list indices [vb, vb + 256) into seg4, one byte each (27-cell stencil): every
+// non-empty segment marks its first index with its number, and a running maximum over the bytes (segments
+// ascend with the index) fills the rest, `last` being the segment in force at vb. About 25 instructions for
+// 256 candidates, where a search per candidate took 20 for each 64.
+__device__ __forceinline__ void fill_segments(uint32_t* seg4, int vb, int seg_off, int seg_cnt, uint32_t& last)
+{
+    const int lane = threadIdx.x;
+    seg4[lane] = 0u;
+    __syncthreads();
+    const int at = seg_off - vb;
+    if (seg_cnt > 0 && (unsigned)at < 256u) reinterpret_cast<uint8_t*>(seg4)[at] = (uint8_t)lane;
+    __syncthreads();
+    const uint32_t w = seg4[lane];
+    uint32_t b0 = w & 255u, b1 = (w >> 8) & 255u, b2 = (w >> 16) & 255u, b3 = w >> 24;
+    b1 = b0 > b1 ? b0 : b1;
+    b2 = b1 > b2 ? b1 : b2;
+    b3 = b2 > b3 ? b2 : b3;
+    uint32_t m = b3;  // inclusive maximum over the lanes
+    auto step = [&](auto ctrl, auto rows) {
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, false);
+        m = m > o ? m : o;
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    before = before > last ? before : last;
+    b0 = before > b0 ? before : b0;
+    b1 = before > b1 ? before : b1;
+    b2 = before > b2 ? before : b2;
+    b3 = before > b3 ? before : b3;
+    seg4[lane] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
+    const uint32_t top = (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
+    last = top > last ? top : last;
+    __syncthreads();
+}
+
+// Keeps the candidates of the supercell's list (of `total` <= kPreCap) that lie within the support radius
+// of its nt <= 64 targets' bounding box B: their entries go to `list`, in list order, the kept index of each
+// target to self_s; returns how many there are. seg4: 64 words for fill_segments. Both pair passes are bound
+// by their vector instructions (3.2 to 3.5 cycles each): segments by table instead of a search, medians
+// instead of two maxima per axis, uniform work on the scalar unit and candidates consecutive in LDS took a
+// density wave from 2,440 to 2,060 of them and a force wave from 3,030 to 2,740; at 2,097,152 particles the
+// density pass went from 0.528 to 0.457 ms and the force pass from 0.70 to 0.68 ms.
 template <int NS>
 __device__ __forceinline__ int prefilter(const NbListT<NS>& L, const WorkBuf& W, const TargetBox& B, int nt,
-                                         int total, int self_v0, float H2, PreList& P, bool& on)
+                                         int total, int self_v0, float H2, uint16_t* list, uint16_t* self_s,
+                                         uint32_t* seg4)
 {
-    on = nt <= 64 && total <= kPreCap;
-    if (!on) return total;
     const int lane = threadIdx.x;
-    const float lx = B.lx, hx = B.hx, ly = B.ly, hy = B.hy, lz = B.lz, hz = B.hz;
     // The test cannot drop a candidate the cull accepts, at any coordinate magnitude: per axis the
     // rounded distance to the box is at most the rounded distance to any target in it (rounding is
     // monotone), and both sums of squares round in the same fma order, so the cull's r2 is never
     // below this d2. The 2^-13 margin on H^2 is kept on top of that.
-    const float H2m = H2 * (1.0f + 1.0f / 8192.0f);
+    const float H2m = B.lx <= B.hx ? H2 * (1.0f + 1.0f / 8192.0f) : -1.0f;  // no targets: nothing is kept
     int count = 0;
-    // four candidates per lane and round, all four records requested before any is tested
+    int seg_off = 0, seg_cnt = 0;  // lane's own segment of the 27
+    uint32_t last = 0;
+    if (NS == 27 && lane < 27) {
+        seg_off = L.off[lane];
+        seg_cnt = L.off[lane + 1] - seg_off;
+    }
+    // four candidates per lane and round, all four records requested before any is tested; lanes past the
+    // end take the last candidate's place and are cut off from what is kept
     for (int vb = 0; vb < total; vb += 256) {
-        float4 q[4];
-        int sg[4];
+        if constexpr (NS == 27) fill_segments(seg4, vb, seg_off, seg_cnt, last);
+        float4 q[4], t[4];
+        int v[4], sg[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int v = vb + 64 * r + lane;
-            sg[r] = 0;
-            q[r] = make_float4(kSentinel, kSentinel, kSentinel, 0.f);
-            if (v < total) {
-                sg[r] = nb_segment(L, v);
-                q[r] = W.P0[L.start[sg[r]] + (v - L.off[sg[r]])];
-            }
+            const int at = vb + 64 * r + lane;
+            v[r] = at < total ? at : total - 1;
+            sg[r] = NS == 27 ? (int)reinterpret_cast<const uint8_t*>(seg4)[v[r] - vb] : nb_segment(L, v[r]);
         }
 #pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = L.t[sg[r]];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (vb + 64 * r < total) q[r] = W.P0[v[r] + __float_as_int(t[r].w)];
+#pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int v = vb + 64 * r + lane;
-            bool keep = false;
-            if (v < total) {
-                const float px = q[r].x + L.sh[sg[r]][0], py = q[r].y + L.sh[sg[r]][1], pz = q[r].z + L.sh[sg[r]][2];
-                const float dx = fmaxf(fmaxf(lx - px, px - hx), 0.0f);
-                const float dy = fmaxf(fmaxf(ly - py, py - hy), 0.0f);
-                const float dz = fmaxf(fmaxf(lz - pz, pz - hz), 0.0f);
-                keep = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < H2m;  // sentinel records: +inf, dropped
-            }
-            const uint64_t b = __ballot(keep);
-            if (keep) {
-                const int sidx = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
-                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-                P.v[sidx] = pre_entry<NS>(v, sg[r]);
-                const unsigned ts = (unsigned)(v - self_v0);
-                if (ts < (unsigned)nt) P.self_s[ts] = (uint16_t)sidx;
+            const int v0 = vb + 64 * r;
+            if (v0 >= total) break;
+            const float px = q[r].x + t[r].x, py = q[r].y + t[r].y, pz = q[r].z + t[r].z;
+            // distance to the box per axis: to the nearest point of it (the median of the coordinate
+            // and the two faces), the same rounded value as the difference to the face
+            const float dx = px - __builtin_amdgcn_fmed3f(px, B.lx, B.hx);
+            const float dy = py - __builtin_amdgcn_fmed3f(py, B.ly, B.hy);
+            const float dz = pz - __builtin_amdgcn_fmed3f(pz, B.lz, B.hz);
+            const bool near = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < H2m;  // sentinel records: +inf, dropped
+            const uint64_t in = total - v0 >= 64 ? ~0ull : (1ull << (total - v0)) - 1ull;
+            const uint64_t b = __ballot(near) & in;
+            const int sidx = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)b, (uint32_t)count));
+            const bool keep = (b >> lane) & 1ull;
+            if (keep) list[sidx] = pre_entry<NS>(v[r], sg[r]);
+            if (v0 + 64 > self_v0 && v0 < self_v0 + nt) {  // the targets' own places
+                const unsigned ts = (unsigned)(v[r] - self_v0);
+                if (keep && ts < (unsigned)nt) self_s[ts] = (uint16_t)sidx;
             }
             count += __popcll(b);
         }
@@ -577,34 +731,30 @@ __device__ __forceinline__ int prefilter(const NbListT<NS>& L, const WorkBuf& W,
     return count;
 }
 
-// Cull lim (<= 32) consecutive lane candidates starting at LDS slot e0 (stride K): bit ii set iff
-// r2 < H2, read off the sign of r2 - H2 (exact: the rounded difference has the sign of the exact
-// one). Returns LSB-first bits.
-__device__ __forceinline__ uint32_t cull32(const float4* __restrict__ sp, int e0, int K, int lim, float xi, float yi,
-                                           float zi, float H2)
+// Cull lim (<= 32) consecutive lane candidates in the LDS slots from sp on: bit ii set iff r2 < H2, read
+// off the sign of r2 - H2 (exact: the rounded difference has the sign of the exact one). Returns
+// LSB-first bits. Candidates go four at a time, all four LDS reads issued before any is used, up to
+// three slots past lim (the caller's LDS array has them; their bits are cut off).
+__device__ __forceinline__ uint32_t cull32(const float4* __restrict__ sp, int lim, float xi, float yi, float zi,
+                                           float H2)
 {
     uint32_t m = 0;
-    if (lim == 32) {
-        // candidates two at a time, both LDS reads issued before either is used: the scheduler
-        // otherwise waits out every read alone to save registers (density pass 1.5% faster)
-#pragma unroll
-        for (int i0 = 0; i0 < 32; i0 += 2) {
-            const float4 q0 = sp[e0 + i0 * K], q1 = sp[e0 + (i0 + 1) * K];
-            __builtin_amdgcn_sched_barrier(0);
-            float dx, dy, dz;
-            const float r2a = geom_r2(xi, yi, zi, q0, dx, dy, dz);
-            m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2a - H2), 31);  // (m << 1) | sign
-            const float r2b = geom_r2(xi, yi, zi, q1, dx, dy, dz);
-            m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2b - H2), 31);
-        }
-        return __builtin_bitreverse32(m);
-    }
-    for (int ii = 0; ii < lim; ++ii) {
+    int n = 0;
+    for (; n < lim; n += 4) {
+        const float4 q0 = sp[n], q1 = sp[n + 1], q2 = sp[n + 2], q3 = sp[n + 3];
+        __builtin_amdgcn_sched_barrier(0);
         float dx, dy, dz;
-        const float r2 = geom_r2(xi, yi, zi, sp[e0 + ii * K], dx, dy, dz);
-        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2 - H2), 31);  // (m << 1) | sign
+        const float r2a = geom_r2(xi, yi, zi, q0, dx, dy, dz);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2a - H2), 31);  // (m << 1) | sign
+        const float r2b = geom_r2(xi, yi, zi, q1, dx, dy, dz);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2b - H2), 31);
+        const float r2c = geom_r2(xi, yi, zi, q2, dx, dy, dz);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2c - H2), 31);
+        const float r2d = geom_r2(xi, yi, zi, q3, dx, dy, dz);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2d - H2), 31);
     }
-    return __builtin_bitreverse32(m) >> (32 - lim);
+    const uint32_t bits = __builtin_bitreverse32(m) >> (32 - n);
+    return lim == 32 ? bits : bits & ((1u << lim) - 1u);
 }
 
 // Staged order of a supercell's candidates in the chunked pair passes. The virtual list (the
@@ -642,14 +792,12 @@ struct StageOrder {
     {
         if (v >= 8 * nfull) return v;
         const int blk = v >> 3, c = cm1 + 1;
-        int i, j;
-        if (blk < rem * c) {
-            i = blk / c;
-            j = blk - i * c;
-        } else {  // only reached when cm1 > 0
-            i = rem + (blk - rem * c) / cm1;
-            j = blk - (i * cm1 + rem);
-        }
+        const bool longrow = blk < rem * c;
+        // short rows are only reached when cm1 > 0
+        const int num = longrow ? blk : blk - rem * c, den = longrow ? c : cm1;
+        const int q = quot(num, den, fast_rcp((float)den));
+        const int i = longrow ? q : rem + q;
+        const int j = num - q * den;
         return 8 * (8 * j + i) + (v & 7);
     }
 };
@@ -657,6 +805,7 @@ struct StageOrder {
 // Lane layout of a supercell-wave: nt targets, K = floor(64/nt) (capped) lanes per target.
 struct LaneMap {
     int K, tpg, tl, k, gfirst, glast;
+    float rK;  // 1 / K
     bool inwave;
 };
 
@@ -664,10 +813,11 @@ __device__ __forceinline__ LaneMap lane_map(int nt, int kmax)
 {
     LaneMap m;
     const int lane = threadIdx.x;
-    int K = nt >= 64 ? 1 : 64 / nt;
+    int K = nt >= 64 ? 1 : uquot(64, nt, fast_rcp((float)nt));
     m.K = K < kmax ? K : kmax;
-    m.tpg = 64 / m.K;
-    m.tl = (int)(((float)lane + 0.5f) * (1.0f / (float)m.K));  // lane / K, exact for lane < 64
+    m.rK = fast_rcp((float)m.K);
+    m.tpg = uquot(64, m.K, m.rK);
+    m.tl = (int)(((float)lane + 0.5f) * m.rK);  // lane / K, exact for lane < 64
     m.k = lane - m.tl * m.K;
     m.inwave = m.tl < m.tpg;
     m.gfirst = m.inwave ? m.tl * m.K : 63;
@@ -675,24 +825,56 @@ __device__ __forceinline__ LaneMap lane_map(int nt, int kmax)
     return m;
 }
 
+// LDS places of a chunk's slots: lane candidate c of sub-lane k at k * stride + c, so that a lane's
+// candidates are consecutive (their addresses are constants off one register in the cull). With few
+// sub-lanes the stride is odd, which keeps them off each other's LDS banks. CAP slots hold
+// K * stride of them and the three that the cull may read past the last.
+struct ChunkMap {
+    int per;     // lane candidates per chunk
+    int stride;  // >= per
+
+    __device__ __forceinline__ ChunkMap(int cap, const LaneMap& m)
+    {
+        stride = uquot(cap - 3, m.K, m.rK);
+        if (m.K <= 8) stride = (stride - 1) | 1;
+        per = stride;
+    }
+    // place of the slot e = c * K + k of a chunk
+    __device__ __forceinline__ int place(int e, const LaneMap& m) const
+    {
+        const int c = (int)(((float)e + 0.5f) * m.rK);  // e / K, exact for e < 2^20
+        return (int)__umul24((unsigned)(e - c * m.K), (unsigned)stride) + c;
+    }
+};
+
 // Whether a supercell-wave keeps its masks: one target group and every lane's candidates fit.
 __device__ __forceinline__ bool masks_fit(int nt, int total, const LaneMap& m, int words = kMaskWords)
 {
-    return nt <= m.tpg && (total + m.K - 1) / m.K <= 32 * words;
+    return nt <= m.tpg && uquot(total + m.K - 1, m.K, m.rK) <= 32 * words;
 }
 
 // The pre-filter's kept list travels from the density pass to the force pass in the top of the
-// supercell's mask row (kMaskWords x 64 words, seen as 16-bit entries): entry 1023 holds the kept
-// count (or kNoList), entries 1022, 1021, ... the kept list indices. With the filter on, masks use at
-// most kMaskWords - 1 words of each lane, so the count never shares a word with mask bits, and the
-// list is stored only where it stays above the words the masks use.
-constexpr uint16_t kNoList = 0xffffu;
-constexpr int kRow16 = kMaskWords * 64 * 2;  // 16-bit entries per mask row
-
-__device__ __forceinline__ bool list_fits(int count, int K)
+// supercell's mask row (kMaskWords x 64 words): the last word holds the kept count (or kNoList), the
+// 16-bit entries lie below it, downwards. With the filter on, masks use at most kMaskWords - 1 words of
+// each lane, so the count never shares a word with mask bits, and the list counts as stored only where it
+// stays above the words the masks use.
+constexpr uint32_t kNoList = 0xffffffffu;
+constexpr int kRowWords = kMaskWords * 64;
+__device__ __forceinline__ uint16_t* row_entry0(uint32_t* row)
 {
-    const int mask_words = ((count + K - 1) / K + 31) / 32;
-    return count <= kRow16 - 1 - 128 * mask_words;
+    return reinterpret_cast<uint16_t*>(row + kRowWords - 1) - 1;  // entry e at [-e]
+}
+// entries 2 d and 2 d + 1 of a row, the first in the low half
+__device__ __forceinline__ uint32_t row_entries(const uint32_t* row, int d)
+{
+    const uint32_t w = row[kRowWords - 2 - d];
+    return (w << 16) | (w >> 16);
+}
+
+__device__ __forceinline__ bool list_fits(int count, int K, float rK)
+{
+    const int mask_words = (uquot(count + K - 1, K, rK) + 31) / 32;
+    return (count + 1) / 2 <= kRowWords - 1 - 64 * mask_words;
 }
 
 // Mask words are indexed by lane candidate c (candidate v = c*K + k of sub-lane k), so the two
@@ -739,10 +921,10 @@ __device__ __forceinline__ uint32_t mask_get(const uint32_t* row, int c0, int li
     return nvalid == 32 ? a : (a & ((1u << nvalid) - 1u));
 }
 
-// Compact the accepted LDS slots of each target's K lanes into lst[gfirst*32 ...) (in sub-lane,
-// then candidate order) and return the target's count; the K lanes then share them round-robin.
+// Compact the accepted LDS slots (first + bit) of each target's K lanes into lst[gfirst*32 ...) (in
+// sub-lane, then candidate order) and return the target's count; the K lanes then share them round-robin.
 template <class LT>
-__device__ __forceinline__ int compact_group(uint32_t msk, int sb, const LaneMap& m, LT* lst)
+__device__ __forceinline__ int compact_group(uint32_t msk, int first, const LaneMap& m, LT* lst)
 {
     const int na = __popc(msk);
     const int incl = wave_incl_scan(na);
@@ -753,7 +935,7 @@ __device__ __forceinline__ int compact_group(uint32_t msk, int sb, const LaneMap
     while (msk) {
         const int ii = __builtin_ctz(msk);
         msk &= msk - 1;
-        lst[wpos++] = (LT)(m.k + (sb + ii) * m.K);
+        lst[wpos++] = (LT)(first + ii);
     }
     return m.inwave ? gtot : 0;
 }
@@ -765,38 +947,62 @@ __device__ __forceinline__ float grad_factor(int kern, float sig, float h)
     return (kern == 2) ? -5.0f * sig / (h * h * h * h * h) : sig / (h * h * h * h);
 }
 
+// x from lane I of the same four-lane quad (DPP quad_perm)
+template <int I>
+__device__ __forceinline__ float quad_bcast(float x)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), I * 0x55, 0xf, 0xf, true));
+}
+template <int I>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, I * 0x55, 0xf, 0xf, true);
+}
+
 // K partial sums of a target combined in lane order (deterministic); then one lane per particle
 // writes rho, the neighbour count and the interaction records of the force pass, and the run's
 // fast-speed maximum (cleaning speed) is raised.
 template <bool MHD>
-__device__ __forceinline__ void density_finish(const RunDev& R, int r, StateBuf& S, WorkBuf& W, const LaneMap& lm,
+__device__ __forceinline__ void density_finish(RunC& R, int r, const StateBuf& S, const WorkBuf& W, const LaneMap& lm,
                                                float acc, uint32_t cnt, bool valid, bool tgt, uint8_t spc,
-                                               uint8_t live, int i, float m_own, float h, float invh, float uu,
+                                               uint8_t live, const Slot& s, float m_own, float h, float uu,
                                                float vx, float vy, float vz, float rho_in, float bx, float by,
                                                float bz, float psi, float gam, int kern)
 {
     const int K = lm.K, k = lm.k;
     const int lane = threadIdx.x;
-    // combine the K partial sums in lane order (deterministic)
     float acc_t = 0.0f;
     uint32_t cnt_t = 0;
-    for (int kk = 0; kk < K; ++kk) {
-        const int src = lm.gfirst + kk < 64 ? lm.gfirst + kk : 63;
-        acc_t += __shfl(acc, src, 64);
-        cnt_t += __shfl(cnt, src, 64);
+    if (K == 4) {  // a target's lanes are one quad: the same additions without the shuffles
+        acc_t += quad_bcast<0>(acc);
+        acc_t += quad_bcast<1>(acc);
+        acc_t += quad_bcast<2>(acc);
+        acc_t += quad_bcast<3>(acc);
+        cnt_t = quad_bcast<0>(cnt) + quad_bcast<1>(cnt) + quad_bcast<2>(cnt) + quad_bcast<3>(cnt);
+    } else {
+        for (int kk = 0; kk < K; ++kk) {
+            const int src = lm.gfirst + kk < 64 ? lm.gfirst + kk : 63;
+            acc_t += __shfl(acc, src, 64);
+            cnt_t += __shfl(cnt, src, 64);
+        }
     }
     // epilogue: one lane per particle writes rho and its interaction records
     float cmax = 0.0f;
     if (k == 0 && valid && is_source(spc, live)) {
 #pragma clang fp contract(off)
         const float sig = R.sigma;
-        const float wfac = sig / (h * h * h);
-        const float gfac = grad_factor(kern, sig, h);
+        // the divisions by powers of h are the run's own constants where the wave's particles have its h
+        float invh = R.inv_h0, wfac = R.wfac0, gfac = R.gfac0;
+        if (__ballot(h != R.h0) != 0) {
+            invh = 1.0f / h;
+            wfac = sig / (h * h * h);
+            gfac = grad_factor(kern, sig, h);
+        }
         float rho;
         if (tgt) {
-            rho = wfac * (acc_t + m_own * R.f0);
-            S.rho[i] = rho;
-            W.nnb[i] = cnt_t;
+            rho = wfac * (acc_t + m_own * kshape0(kern));
+            s.col(S.rho) = rho;
+            s.col(W.nnb) = cnt_t;
         } else {
             rho = rho_in;
         }
@@ -808,20 +1014,19 @@ __device__ __forceinline__ void density_finish(const RunDev& R, int r, StateBuf&
         const float pr = (P + 0.5f * B2) * bdr;
         const float psr = psi * bdr;
         const float c = sqrtf((gam * P + B2) * invrho);
-        W.P1[i] = make_float4(vx, vy, vz, c);
-        W.P2[i] = make_float4(h, invh, gfac, ph);
-        W.P3[i] = make_float4(pr, 0.5f * rho, bdr, psr);
-        if (MHD) W.P4[i] = make_float4(bx, by, bz, psi);
+        s.rec(W.P1) = make_float4(vx, vy, vz, c);
+        s.rec(W.P2) = make_float4(h, invh, gfac, ph);
+        s.rec(W.P3) = make_float4(pr, 0.5f * rho, bdr, psr);
+        if (MHD) s.rec(W.P4) = make_float4(bx, by, bz, psi);
         if (tgt) cmax = c;
     }
-    if (k == 0 && valid && !tgt) W.nnb[i] = 0;
-    if (MHD && R.mhd && R.cleaning) {
-        for (int off = 32; off >= 1; off >>= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, off, 64));
+    if (k == 0 && valid && !tgt) s.col(W.nnb) = 0;
+    if (MHD && run_mhd(R.flags) && run_cleaning(R.flags)) {
+        const uint32_t bits = dpp_max_u32(__float_as_uint(cmax));
         // every wave of the run targets this one word: test before the atomic, so that only a
         // wave holding a new maximum pays for one (the value only grows, so a stale read costs
         // at most a redundant atomic)
-        if (lane == 0 && cmax > 0.0f) {
-            const uint32_t bits = __float_as_uint(cmax);
+        if (lane == 0 && bits != 0u) {
             if (bits > __atomic_load_n(&W.chbits[r], __ATOMIC_RELAXED)) atomicMax(&W.chbits[r], bits);
         }
     }
@@ -831,111 +1036,140 @@ __device__ __forceinline__ void density_finish(const RunDev& R, int r, StateBuf&
 // density pass: cull of the 27-supercell candidates staged in LDS, density sum, candidate masks,
 // and the per-particle interaction records of the force pass
 // ------------------------------------------------------------------------------------------------
-// With the Wendland kernel the pass fits 64 VGPRs without spilling: 8 waves per SIMD instead of 7,
-// 5% faster on the 2M-particle turbulence step. The other kernels keep the compiler's choice
-// (a cap spills them), as do the balanced pass and the 125-cell stencil with 256-candidate chunks,
-// whose LDS allows 6.
+// LDS of a density wave (27-cell stencil, 256 slots: 4,768 bytes, so that 32 waves fit a compute unit). sp
+// holds the staged candidates, its top the pre-filter's kept list while there is one (160 slots are left for
+// a chunk then), and its first slots the segment table while the pre-filter runs. Staging the kept candidates
+// straight from the filter, without their list, needs room for all of them (236 on average in a turbulent
+// state, 330 at the 95th percentile) and cost more in occupancy than the second pass over their records:
+// 0.476 / 0.504 ms with 320 / 384 slots at 7 / 6 waves per SIMD against 0.450 ms at 2,097,152 particles.
+template <int CH, int RMAX>
+struct DensityLds {
+    NbListR<RMAX> L;
+    float4 sp[CH];
+    uint16_t self_s[64];
+};
+constexpr int kListSlots = kPreCap * 2 / 16;  // slots that the kept list takes
+
 template <int CH, bool MIXED, bool MHD, int KT, int RMAX>
-__device__ __forceinline__ void density_wave(int vb, const RunDev* __restrict__ runs, int nruns, int ncell_tot,
-                                             int nblk_total, StateBuf& S, WorkBuf& W, int kmax, NbListR<RMAX>& L,
-                                             float4 (&sp)[CH], PreList& P)
+__device__ __forceinline__ void density_wave(int vb, DensityLds<CH, RMAX>& lds)
 {
+    const PairArgs& args = pair_args();
+    const StateBuf& S = args.S;
+    const WorkBuf& W = args.W;
+    const RunDev* const runs = args.runs;
     constexpr int NS = RMAX == 1 ? 27 : 125;
-    const int cell = xcd_cell(vb, nblk_total, ncell_tot);
+    static_assert(CH - kListSlots >= 67, "a chunk beside the kept list needs a slot per lane and the cull's three");
+    NbListR<RMAX>& L = lds.L;
+    float4(&sp)[CH] = lds.sp;
+    const int cell = xcd_cell(vb, args.nblk_total, args.ncell_tot);
     if (cell < 0) return;
-    const int t0 = (int)W.cs[cell];
-    const int nt = (int)W.cs[cell + 1] - t0;
+    const int t0 = uniform((int)W.cs[cell]);
+    const int nt = uniform((int)W.cs[cell + 1]) - t0;
     if (nt == 0) return;
-    const int r = find_run_by_cell(runs, nruns, cell);
-    const RunDev& R = runs[r];
+    const int r = find_run_by_cell(runs, args.nruns, cell);
+    RunC& R = ((RunC*)runs)[r];
     // the targets' box inputs are requested before the neighbour list, so their loads overlap the list's
     const TargetBoxInput box_in = nt <= 64 ? target_box_load(S, W, t0, nt) : TargetBoxInput{};
-    build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L);
-    const int self_v0 = L.off[self_segment<RMAX>(R)];
-    bool pre;
-    const int total = prefilter<NS>(L, W, nt <= 64 ? target_box(box_in, nt) : TargetBox{}, nt, L.off[NS], self_v0,
-                                    R.H2, P, pre);  // staged candidates
-    const StageOrder so(total);
+    int self_v0;
+    const int all = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
     const int lane = threadIdx.x;
-    const LaneMap lm = lane_map(nt, kmax);
+    const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
-    const int per = CH / K;   // lane candidates per chunk
-    const int chk = per * K;  // staged entries per chunk (a multiple of K)
-    const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
+    uint32_t* const row = W.nbmask != nullptr ? W.nbmask + (size_t)cell * kRowWords : nullptr;
+    // supercells of more than 64 particles or a longer list are not filtered
+    const bool pre = nt <= 64 && all <= kPreCap;
+    uint16_t* const list = reinterpret_cast<uint16_t*>(sp + CH - kListSlots);
+    const ChunkMap cm(pre ? CH - kListSlots : CH, lm);
+    int total = all;  // staged candidates
+    if (pre)
+        total = prefilter<NS>(L, W, target_box(box_in, nt), nt, all, self_v0, R.H2, list, lds.self_s,
+                              reinterpret_cast<uint32_t*>(sp));
+    const StageOrder so(total);
+    const int chk = cm.per * K;  // staged entries per chunk (a multiple of K)
+    const int kern = KT >= 0 ? KT : run_kernel(R.flags);  // compile-time when every run uses one kernel
     const float H2 = R.H2;
     const float gam = R.gamma;
     // no mask table: density only; with the filter on the top word of each lane carries the kept list
-    const bool keep = masks_fit(nt, total, lm, pre ? kMaskWords - 1 : kMaskWords) && W.nbmask != nullptr;
+    const bool keep = masks_fit(nt, total, lm, pre ? kMaskWords - 1 : kMaskWords) && row != nullptr;
     MaskWriter mw;
-    mw.row = W.nbmask + (size_t)cell * (kMaskWords * 64) + lane;
+    mw.row = row + lane;
     mw.pend = 0;
     mw.pend_w = -1;
-    mw.wlim = ((total + K - 1) / K + 31) / 32;  // the words the lane's candidates need
+    mw.wlim = (uquot(total + K - 1, K, lm.rK) + 31) / 32;  // the words the lane's candidates need
 
     for (int tg = 0; tg < nt; tg += lm.tpg) {
-        const int t = tg + lm.tl;
-        const bool valid = lm.inwave && t < nt;
-        const int i = t0 + (valid ? t : 0);
-        const uint8_t live = S.mask[i], spc = S.species[i];
+        const int tt = tg + lm.tl;
+        const bool valid = lm.inwave && tt < nt;
+        // t0 made opaque in the loop (one round for most cells): otherwise the bases of all the columns
+        // are formed ahead of it and no scalar registers are left
+        int t0l = t0;
+        asm volatile("" : "+s"(t0l));
+        const Slot s(t0l, valid ? (uint32_t)tt : 0u);
+        const uint8_t live = s.col(S.mask), spc = s.col(S.species);
         const bool tgt = valid && is_target(spc, live);
-        const float4 own = W.P0[i];
-        const float h = S.h[i];
+        const float4 own = s.rec(W.P0);
+        const float h = s.col(S.h);
         // inputs of the epilogue, loaded early so their latency overlaps the cull
-        const float uu = S.u[i];
-        const float vx = S.vel[0][i], vy = S.vel[1][i], vz = S.vel[2][i];
-        const float rho_in = S.rho[i];
+        const float uu = s.col(S.u);
+        const float vx = s.col(S.vel[0]), vy = s.col(S.vel[1]),
+                    vz = s.col(S.vel[2]);
+        const float rho_in = s.col(S.rho);
         float bx = 0.f, by = 0.f, bz = 0.f, psi = 0.f;
-        if (MHD && R.mhd) {
-            bx = S.B[0][i];
-            by = S.B[1][i];
-            bz = S.B[2][i];
-            psi = S.psi[i];
+        if (MHD && run_mhd(R.flags)) {
+            bx = s.col(S.B[0]);
+            by = s.col(S.B[1]);
+            bz = s.col(S.B[2]);
+            psi = s.col(S.psi);
         }
-        const float invh = 1.0f / h;
-        const int self_u = tgt ? so.slot(pre ? (int)P.self_s[t] : self_v0 + t) : -1;  // staged slot of the self pair
+        float invh = R.inv_h0;
+        if (__ballot(h != R.h0) != 0) invh = 1.0f / h;
+        // the lane candidate that is the self pair: its staged slot is this lane's or no lane candidate
+        int self_c = -1;
+        if (tgt) {
+            const int self_u = so.slot(pre ? (int)lds.self_s[tt] : self_v0 + tt);
+            const int c = quot(self_u, K, lm.rK);
+            self_c = self_u - c * K == k ? c : -1;
+        }
         float acc = 0.0f;
         uint32_t cnt = 0;
+        const float4* const mine = sp + __umul24((unsigned)k, (unsigned)cm.stride);  // this lane's slots
 
-        for (int base = 0; base < total; base += chk) {
-            for (int e = lane; e < chk; e += 64) {
+        for (int base = 0, cbase = 0; base < total; base += chk, cbase += cm.per) {
+            // lane slots of this chunk that hold candidates (the most any lane has): the last chunk's
+            // padding is not culled
+            const int left = total - base < chk ? total - base : chk;
+            const int nval = uquot(left + K - 1, K, lm.rK);
+            for (int e = lane; e < nval * K; e += 64) {
                 const int u = base + e;
                 float4 p = make_float4(kSentinel, kSentinel, kSentinel, 0.0f);
                 if (u < total) {
-                    int v, sg;
-                    staged_candidate<NS>(L, P, pre, so.list_index(u), v, sg);
-                    p = W.P0[L.start[sg] + (v - L.off[sg])];
-                    p.x += L.sh[sg][0];
-                    p.y += L.sh[sg][1];
-                    p.z += L.sh[sg][2];
+                    float4 t4;
+                    const int li = so.list_index(u);
+                    const int j = pre ? kept_candidate(L, list[li], t4) : list_candidate(L, li, t4);
+                    p = W.P0[j];
+                    p.x += t4.x;
+                    p.y += t4.y;
+                    p.z += t4.z;
                 }
-                sp[e] = p;
+                sp[cm.place(e, lm)] = p;
             }
             __syncthreads();
-            const int cbase = base / K;
-            // lane slots of this chunk that hold candidates (the most any lane has): the last chunk's
-            // padding is not culled
-            const int nval = ((total - base < chk ? total - base : chk) + K - 1) / K;
             for (int sb = 0; sb < nval; sb += 32) {
                 const int lim = nval - sb < 32 ? nval - sb : 32;
-                uint32_t msk = cull32(sp, k + sb * K, K, lim, own.x, own.y, own.z, H2);
+                uint32_t msk = cull32(mine + sb, lim, own.x, own.y, own.z, H2);
                 // the self pair (r2 = 0) passes the cull: drop it here; its density term is the
                 // self term m_i W(0, h_i) added below, as DensityInitSelf does
-                const int sc = self_u - k;
-                if (sc >= 0 && sc % K == 0) {
-                    const int bit = sc / K - cbase - sb;
-                    if (bit >= 0 && bit < lim) msk &= ~(1u << bit);
-                }
+                const unsigned bit = (unsigned)(self_c - cbase - sb);
+                if (bit < (unsigned)lim) msk &= ~(1u << bit);
                 if (!tgt) msk = 0;
                 if (keep) mw.put(msk, cbase + sb, lim);
                 cnt += (uint32_t)__popc(msk);
                 // each lane sums its own accepted candidates (the density pairs are too cheap for
                 // sharing them among a target's lanes to pay for the compaction)
-                const int kb = (int)sizeof(float4) * K;
-                const int eb0 = (int)sizeof(float4) * (k + sb * K);  // byte offset of bit 0's slot
                 while (msk) {
                     const int ii = __builtin_ctz(msk);
                     msk &= msk - 1;
-                    const float4 p = lds_at(sp, (int)__umul24((unsigned)ii, (unsigned)kb) + eb0);
+                    const float4 p = lds_at(mine + sb, ii * (int)sizeof(float4));
                     float dx, dy, dz;
                     const float r2 = geom_r2(own.x, own.y, own.z, p, dx, dy, dz);
                     acc += p.w * kshape(kern, fast_sqrt(r2) * invh);
@@ -944,38 +1178,33 @@ __device__ __forceinline__ void density_wave(int vb, const RunDev* __restrict__ 
             __syncthreads();
         }
         if (keep) mw.flush();
-        density_finish<MHD>(R, r, S, W, lm, acc, cnt, valid, tgt, spc, live, i, own.w, h, invh, uu, vx, vy, vz,
-                            rho_in, bx, by, bz, psi, gam, kern);
+        density_finish<MHD>(R, r, S, W, lm, acc, cnt, valid, tgt, spc, live, s, own.w, h, uu, vx, vy, vz, rho_in,
+                            bx, by, bz, psi, gam, kern);
     }
     // the kept list for the force pass, stored last: stores count in the same wait counter as the
     // loads, so stored earlier they would delay every later wait for the staging loads
-    if (pre && W.nbmask != nullptr) {
-        uint16_t* row16 = reinterpret_cast<uint16_t*>(W.nbmask + (size_t)cell * (kMaskWords * 64));
-        const bool store = keep && list_fits(total, K);
+    if (pre && row != nullptr) {
+        const bool store = keep && list_fits(total, K, lm.rK);
         if (store)
-            for (int e = lane; e < total; e += 64) row16[kRow16 - 2 - e] = P.v[e];
-        if (lane == 0) row16[kRow16 - 1] = store ? (uint16_t)total : kNoList;
+            for (int e = lane; e < total; e += 64) *(row_entry0(row) - e) = list[e];
+        if (lane == 0) row[kRowWords - 1] = store ? (uint32_t)total : kNoList;
     }
 }
 
 template <int CH, bool MIXED, bool MHD, int KT, int RMAX = 1, bool GRID = false>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu((KT == 2 && !(RMAX == 2 && CH > 128)) ? 8 : 1)))  // KT 2: Wendland
-void k_density(const RunDev* __restrict__ runs, int nruns, int ncell_tot, int nblk_total, StateBuf S, WorkBuf W,
-               int kmax)
+__attribute__((amdgpu_waves_per_eu(KT == 2 && RMAX == 1 ? 8 : 1, 8)))  // KT 2: Wendland
+void k_density(PairArgs)
 {
-    __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[CH];
-    __shared__ PreList P;
+    __shared__ DensityLds<CH, RMAX> lds;
     if constexpr (GRID) {
         // a persistent grid: each wave walks the supercells at a stride of the grid (a multiple
         // of 8, so every cell a wave visits belongs to its own XCD's range)
-        for (int vb = blockIdx.x; vb < nblk_total; vb += gridDim.x)
-            density_wave<CH, MIXED, MHD, KT, RMAX>(vb, runs, nruns, ncell_tot, nblk_total, S, W, kmax, L, sp, P);
+        for (int vb = blockIdx.x; vb < pair_args().nblk_total; vb += gridDim.x)
+            density_wave<CH, MIXED, MHD, KT, RMAX>(vb, lds);
     } else {
         // one supercell per wave
-        density_wave<CH, MIXED, MHD, KT, RMAX>((int)blockIdx.x, runs, nruns, ncell_tot, nblk_total, S, W, kmax, L,
-                                               sp, P);
+        density_wave<CH, MIXED, MHD, KT, RMAX>((int)blockIdx.x, lds);
     }
 }
 
@@ -995,10 +1224,14 @@ struct PairConst {
     float va, vb;             // alpha / 2 and beta of the viscosity
     float h, invh, gfac, e;   // ONE_H: the run's one smoothing length, 1/h, gradient factor and 0.01 h^2
 
-    __device__ __forceinline__ PairConst(const RunDev& R, int kern_, float h_, float gfac_)
+    __device__ __forceinline__ PairConst(RunC& R, int kern_, float h_)
         : kern(kern_), beta(R.beta), va(R.alpha > 0.0f ? 0.5f * R.alpha : 0.0f), vb(R.alpha > 0.0f ? R.beta : 0.0f),
-          h(h_), invh(1.0f / h_), gfac(gfac_), e((0.01f * h_) * h_)
+          h(h_), invh(R.inv_h0), gfac(R.gfac0), e((0.01f * h_) * h_)
     {
+        if (uniform(__float_as_int(h_)) != __float_as_int(R.h0)) {
+            invh = 1.0f / h_;
+            gfac = grad_factor(kern_, R.sigma, h_);
+        }
     }
 };
 
@@ -1074,8 +1307,8 @@ __device__ __forceinline__ void force_pair(const float4& o0, const float4& o1, c
 
 // One target's derivatives, signal speed and div B from its summed pair terms T.
 template <bool MHD>
-__device__ __forceinline__ void force_write(const RunDev& R, WorkBuf& W, const ForceAcc& T, int i, const float4& o1,
-                                            const float4& o2, const float4& o3, const float4& o4, bool mhd,
+__device__ __forceinline__ void force_write(RunC& R, const WorkBuf& W, const ForceAcc& T, const Slot& s,
+                                            const float4& o1, const float4& o2, const float4& o3, const float4& o4, bool mhd,
                                             bool clean, float borve, float ch)
 {
     const float rho = 2.0f * o3.y;
@@ -1087,11 +1320,11 @@ __device__ __forceinline__ void force_write(const RunDev& R, WorkBuf& W, const F
         ay = ay + T.TBy + o4.y * tcoef;
         az = az + T.TBz + o4.z * tcoef;
     }
-    W.dvdt[0][i] = ax;
-    W.dvdt[1][i] = ay;
-    W.dvdt[2][i] = az;
-    W.dudt[i] = o2.w * T.DV + 0.5f * T.AVU;
-    W.vsig[i] = fmaxf(2.0f * o1.w, T.vmax);
+    s.col(W.dvdt[0]) = ax;
+    s.col(W.dvdt[1]) = ay;
+    s.col(W.dvdt[2]) = az;
+    s.col(W.dudt) = o2.w * T.DV + 0.5f * T.AVU;
+    s.col(W.vsig) = fmaxf(2.0f * o1.w, T.vmax);
     if (MHD && mhd) {
         const float divB = -T.DB * invrho;
         const float divv = -T.DV * invrho;
@@ -1106,11 +1339,11 @@ __device__ __forceinline__ void force_write(const RunDev& R, WorkBuf& W, const F
             const float psi = o4.w;
             dpsi = -ch * ch * divB - psi * R.clean_sigma * ch * o2.y - 0.5f * psi * divv;
         }
-        W.dbdt[0][i] = dbx;
-        W.dbdt[1][i] = dby;
-        W.dbdt[2][i] = dbz;
-        W.dpsidt[i] = dpsi;
-        W.divb[i] = divB;
+        s.col(W.dbdt[0]) = dbx;
+        s.col(W.dbdt[1]) = dby;
+        s.col(W.dbdt[2]) = dbz;
+        s.col(W.dpsidt) = dpsi;
+        s.col(W.divb) = divB;
     }
 }
 
@@ -1127,8 +1360,8 @@ __device__ __forceinline__ float row_shr(float x)
 // it) leave the target's total in its last lane; other K take the shuffles of each lane's partial
 // in lane order to every lane of the target.
 template <bool MHD>
-__device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const LaneMap& lm, ForceAcc& A, bool tgt,
-                                             int i, const float4& o1, const float4& o2, const float4& o3,
+__device__ __forceinline__ void force_finish(RunC& R, const WorkBuf& W, const LaneMap& lm, ForceAcc& A, bool tgt,
+                                             const Slot& s, const float4& o1, const float4& o2, const float4& o3,
                                              const float4& o4, bool mhd, bool clean, float borve, float ch)
 {
     const int K = lm.K, k = lm.k;
@@ -1139,7 +1372,7 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
 #pragma unroll
         for (int f = 0; f < 12; ++f) v[5 + f] = m[f];
     }
-    float s[NF];
+    float sum[NF];
     float vm;
     bool writer;
     if (K == 1 || K == 2 || K == 4 || K == 8 || K == 16) {
@@ -1155,7 +1388,7 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
         if (K >= 8) step(std::integral_constant<int, 4>{});
         if (K >= 16) step(std::integral_constant<int, 8>{});
 #pragma unroll
-        for (int f = 0; f < NF; ++f) s[f] = v[f];
+        for (int f = 0; f < NF; ++f) sum[f] = v[f];
         vm = A.vmax;
         writer = k == K - 1;
     } else {
@@ -1163,7 +1396,7 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
         // of one lane step are fetched together, so a step's shuffles overlap instead of each waiting
         // for the last.
 #pragma unroll
-        for (int f = 0; f < NF; ++f) s[f] = 0.0f;
+        for (int f = 0; f < NF; ++f) sum[f] = 0.0f;
         vm = 0.0f;
         for (int kk = 0; kk < K; ++kk) {
             const int src = lm.gfirst + kk < 64 ? lm.gfirst + kk : 63;
@@ -1172,33 +1405,33 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
             for (int f = 0; f < NF; ++f) t[f] = __shfl(v[f], src, 64);
             const float tm = __shfl(A.vmax, src, 64);
 #pragma unroll
-            for (int f = 0; f < NF; ++f) s[f] += t[f];
+            for (int f = 0; f < NF; ++f) sum[f] += t[f];
             vm = fmaxf(vm, tm);
         }
         writer = k == 0;
     }
     ForceAcc& T = A;
-    T.ax = s[0];
-    T.ay = s[1];
-    T.az = s[2];
-    T.DV = s[3];
-    T.AVU = s[4];
+    T.ax = sum[0];
+    T.ay = sum[1];
+    T.az = sum[2];
+    T.DV = sum[3];
+    T.AVU = sum[4];
     T.vmax = vm;
     if constexpr (MHD) {
-        T.Ti = s[5];
-        T.Tj = s[6];
-        T.TBx = s[7];
-        T.TBy = s[8];
-        T.TBz = s[9];
-        T.VBx = s[10];
-        T.VBy = s[11];
-        T.VBz = s[12];
-        T.DB = s[13];
-        T.PSx = s[14];
-        T.PSy = s[15];
-        T.PSz = s[16];
+        T.Ti = sum[5];
+        T.Tj = sum[6];
+        T.TBx = sum[7];
+        T.TBy = sum[8];
+        T.TBz = sum[9];
+        T.VBx = sum[10];
+        T.VBy = sum[11];
+        T.VBz = sum[12];
+        T.DB = sum[13];
+        T.PSx = sum[14];
+        T.PSy = sum[15];
+        T.PSz = sum[16];
     }
-    if (writer && tgt) force_write<MHD>(R, W, T, i, o1, o2, o3, o4, mhd, clean, borve, ch);
+    if (writer && tgt) force_write<MHD>(R, W, T, s, o1, o2, o3, o4, mhd, clean, borve, ch);
 }
 
 // Records staged per neighbour: P0, P1, P3, P4 with MHD fields, and P2 unless the run has one smoothing
@@ -1206,125 +1439,145 @@ __device__ __forceinline__ void force_finish(const RunDev& R, WorkBuf& W, const 
 template <bool MHD, bool ONE_H>
 constexpr int kForcePlanes = 3 + (MHD ? 1 : 0) + (ONE_H ? 0 : 1);
 
+// LDS slots of a force chunk: CH, the odd-stride rounding of ChunkMap and the cull's three.
+template <int CH>
+constexpr int kForceSlots = CH + 8;
+
 template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX, bool ONE_H = false>
-__device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ runs, int nruns, int ncell_tot,
-                                            int nblk_total, StateBuf& S, WorkBuf& W, int kmax, NbListR<RMAX>& L,
-                                            float4 (&sp)[kForcePlanes<MHD, ONE_H>][CH], ListT<CH> (&lst)[BAL == 1 ? 64 * 32 : 1],
-                                            PreList& P)
+__device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
+                                            float4 (&sp)[kForcePlanes<MHD, ONE_H>][kForceSlots<CH>],
+                                            ListT<CH> (&lst)[BAL == 1 ? 64 * 32 : 1], PreList& P)
 {
+    const PairArgs& args = pair_args();
+    const StateBuf& S = args.S;
+    const WorkBuf& W = args.W;
+    const RunDev* const runs = args.runs;
     constexpr int NS = RMAX == 1 ? 27 : 125;
-    const int cell = xcd_cell(vb, nblk_total, ncell_tot);
+    const int cell = xcd_cell(vb, args.nblk_total, args.ncell_tot);
     if (cell < 0) return;
-    const int t0 = (int)W.cs[cell];
-    const int nt = (int)W.cs[cell + 1] - t0;
+    const int t0 = uniform((int)W.cs[cell]);
+    const int nt = uniform((int)W.cs[cell + 1]) - t0;
     if (nt == 0) return;
-    const int r = find_run_by_cell(runs, nruns, cell);
-    const RunDev& R = runs[r];
+    const int r = find_run_by_cell(runs, args.nruns, cell);
+    RunC& R = ((RunC*)runs)[r];
     const int lane = threadIdx.x;
-    // the density pass's kept set, stored in the mask row: its count and first 256 entries are
-    // requested before the neighbour list is built, so their loads overlap its cell-start loads
-    // (they are used only if this step's filter applies to the supercell, which the list decides)
-    const uint16_t* row16 =
-        W.nbmask != nullptr ? reinterpret_cast<const uint16_t*>(W.nbmask + (size_t)cell * (kMaskWords * 64)) : nullptr;
-    int n_row = kNoList;
-    uint16_t head[4] = {0, 0, 0, 0};
-    if (row16 != nullptr && nt <= 64) {
-        n_row = row16[kRow16 - 1];
+    // the density pass's kept set, stored in the mask row: its count, its first 256 entries and the lane's
+    // first 64 mask bits are requested before the neighbour list is built, so their loads overlap its
+    // cell-start loads (they are used only if this step's filter and masks apply to the supercell, which
+    // the list decides)
+    const uint32_t* row = W.nbmask + (size_t)cell * kRowWords;
+    uint32_t n_row = kNoList, head[2] = {0, 0};
+    if (nt <= 64) {
+        n_row = row[kRowWords - 1];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) head[q] = row16[kRow16 - 2 - (lane + 64 * q)];
+        for (int q = 0; q < 2; ++q) head[q] = row_entries(row, lane + 64 * q);
     }
-    build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L);
-    const int self_v0 = L.off[self_segment<RMAX>(R)];
-    const LaneMap lm = lane_map(nt, kmax);
+    const uint32_t* const mrow = row + lane;
+    const uint64_t m01 = ((uint64_t)mrow[64] << 32) | mrow[0];
+    int self_v0;
+    const int all = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
+    const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
     // read back where the density pass stored it, else recomputed
-    bool pre = nt <= 64 && L.off[NS] <= kPreCap;
-    bool stored = false;
-    int total = L.off[NS];
-    if (pre && row16 != nullptr && n_row != kNoList) {
+    const bool pre = nt <= 64 && all <= kPreCap;
+    int total = all;
+    const int n_kept = uniform((int)n_row);
+    if (pre && (uint32_t)n_kept != kNoList) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (lane + 64 * q < n_row) P.v[lane + 64 * q] = head[q];
-        for (int e = lane + 256; e < n_row; e += 64) P.v[e] = row16[kRow16 - 2 - e];
+        for (int q = 0; q < 2; ++q)
+            if (2 * (lane + 64 * q) < n_kept) P.v2[lane + 64 * q] = head[q];
+        for (int d = lane + 128; 2 * d < n_kept; d += 64) P.v2[d] = row_entries(row, d);
         __syncthreads();
-        total = n_row;
-        stored = true;
+        total = n_kept;
+    } else if (pre) {
+        total = prefilter<NS>(L, W, target_box(target_box_load(S, W, t0, nt), nt), nt, all, self_v0, R.H2, P.v,
+                              P.self_s, P.seg4);
     }
-    if (!stored)
-        total = prefilter<NS>(L, W, pre ? target_box(target_box_load(S, W, t0, nt), nt) : TargetBox{}, nt, total,
-                              self_v0, R.H2, P, pre);
     const StageOrder so(total);  // the density pass's staged order: its masks replay slot by slot
-    const int per = CH / K;
-    const int chk = per * K;
-    const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
+    const ChunkMap cm(kForceSlots<CH>, lm);
+    const int per_lane = uquot(total + K - 1, K, lm.rK);
+    const int kern = KT >= 0 ? KT : run_kernel(R.flags);  // compile-time when every run uses one kernel
     const float H2 = R.H2;
     const float h_own = S.h[t0];  // the run's one smoothing length (ONE_H)
-    const PairConst pc(R, kern, h_own, grad_factor(kern, R.sigma, h_own));
-    const bool mhd = MHD && R.mhd;
-    const bool clean = mhd && R.cleaning;
+    const PairConst pc(R, kern, h_own);
+    const bool mhd = MHD && run_mhd(R.flags);
+    const bool clean = mhd && run_cleaning(R.flags);
     const float borve = mhd ? R.borve : 0.0f;
     const float ch = __uint_as_float(W.chbits[r]);
     const bool keep = masks_fit(nt, total, lm, pre ? kMaskWords - 1 : kMaskWords);
-    const int per_lane = (total + K - 1) / K;
-    const uint32_t* mrow = W.nbmask + (size_t)cell * (kMaskWords * 64) + lane;
+    // as few chunks as the slots allow, of about equal size: a chunk's pair loop waits for its busiest lane,
+    // so a short last chunk would waste rounds
+    const int nch = uquot(per_lane + cm.per - 1, cm.per, fast_rcp((float)cm.per));
+    const int per = uquot(per_lane + nch - 1, nch, fast_rcp((float)nch));
+    const int chk = per * K;
 
     for (int tg = 0; tg < nt; tg += lm.tpg) {
-        const int t = tg + lm.tl;
-        const bool valid = lm.inwave && t < nt;
-        const int i = t0 + (valid ? t : 0);
-        const bool tgt = valid && is_target(S.species[i], S.mask[i]);
-        const float4 o0 = W.P0[i], o1 = W.P1[i], o3 = W.P3[i];
+        const int tt = tg + lm.tl;
+        const bool valid = lm.inwave && tt < nt;
+        // t0 made opaque in the loop (one round for most cells): otherwise the bases of all the columns
+        // are formed ahead of it and no scalar registers are left
+        int t0l = t0;
+        asm volatile("" : "+s"(t0l));
+        const Slot s(t0l, valid ? (uint32_t)tt : 0u);
+        const bool tgt = valid && is_target(s.col(S.species), s.col(S.mask));
+        const float4 o0 = s.rec(W.P0), o1 = s.rec(W.P1), o3 = s.rec(W.P3);
         float4 o2 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (!ONE_H) o2 = W.P2[i];
+        if constexpr (!ONE_H) o2 = s.rec(W.P2);
         float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (MHD) o4 = W.P4[i];
-        // the self slot is needed only where the pass culls (a stored list implies stored masks)
-        const int self_u = tgt && !keep ? so.slot(pre ? (int)P.self_s[t] : self_v0 + t) : -1;
+        if (MHD) o4 = s.rec(W.P4);
+        // the lane candidate that is the self pair is needed only where the pass culls (a stored list
+        // implies stored masks)
+        int self_c = -1;
+        if (tgt && !keep) {
+            const int self_u = so.slot(pre ? (int)P.self_s[tt] : self_v0 + tt);
+            const int c = quot(self_u, K, lm.rK);
+            self_c = self_u - c * K == k ? c : -1;
+        }
         ForceAcc A = {};
+        const int first = (int)__umul24((unsigned)k, (unsigned)cm.stride);  // this lane's slots
 
-        for (int base = 0; base < total; base += chk) {
-            for (int e = lane; e < chk; e += 64) {
-                const int u = base + e;
+        for (int base = 0, cbase = 0; base < total; base += chk, cbase += per) {
+            const int left = total - base < chk ? total - base : chk;
+            const int nval = uquot(left + K - 1, K, lm.rK);
+            for (int e = lane; e < nval * K; e += 64) {
+                const int u = base + e, at = cm.place(e, lm);
                 if (u < total) {
-                    int v, sg;
-                    staged_candidate<NS>(L, P, pre, so.list_index(u), v, sg);
-                    const int j = L.start[sg] + (v - L.off[sg]);
+                    float4 t4;
+                    const int li = so.list_index(u);
+                    const int j = pre ? kept_candidate(L, P.v[li], t4) : list_candidate(L, li, t4);
                     float4 p = W.P0[j];
-                    p.x += L.sh[sg][0];
-                    p.y += L.sh[sg][1];
-                    p.z += L.sh[sg][2];
-                    sp[0][e] = p;
-                    sp[1][e] = W.P1[j];
-                    sp[2][e] = W.P3[j];
-                    if constexpr (MHD) sp[3][e] = W.P4[j];
-                    if constexpr (!ONE_H) sp[MHD ? 4 : 3][e] = W.P2[j];
+                    p.x += t4.x;
+                    p.y += t4.y;
+                    p.z += t4.z;
+                    sp[0][at] = p;
+                    sp[1][at] = W.P1[j];
+                    sp[2][at] = W.P3[j];
+                    if constexpr (MHD) sp[3][at] = W.P4[j];
+                    if constexpr (!ONE_H) sp[MHD ? 4 : 3][at] = W.P2[j];
                 } else {
-                    sp[0][e] = make_float4(kSentinel, kSentinel, kSentinel, 0.0f);
+                    sp[0][at] = make_float4(kSentinel, kSentinel, kSentinel, 0.0f);
                 }
             }
             __syncthreads();
-            const int cbase = base / K;
-            for (int sb = 0; sb < per; sb += 32) {
-                const int lim = per - sb < 32 ? per - sb : 32;
+            for (int sb = 0; sb < nval; sb += 32) {
+                const int lim = nval - sb < 32 ? nval - sb : 32;
+                const int c0 = cbase + sb;
                 uint32_t msk;
                 if (keep) {
-                    msk = mask_get(mrow, cbase + sb, lim, per_lane);
+                    if (c0 + lim <= 64) msk = (uint32_t)(m01 >> c0) & (0xffffffffu >> (32 - lim));
+                    else msk = mask_get(mrow, c0, lim, per_lane);
                 } else {
-                    msk = cull32(sp[0], k + sb * K, K, lim, o0.x, o0.y, o0.z, H2);
-                    const int sc = self_u - k;  // the self pair adds exact zeros; drop it anyway
-                    if (sc >= 0 && sc % K == 0) {
-                        const int bit = sc / K - cbase - sb;
-                        if (bit >= 0 && bit < lim) msk &= ~(1u << bit);
-                    }
+                    msk = cull32(sp[0] + first + sb, lim, o0.x, o0.y, o0.z, H2);
+                    const unsigned bit = (unsigned)(self_c - c0);  // the self pair adds exact zeros; drop it anyway
+                    if (bit < (unsigned)lim) msk &= ~(1u << bit);
                 }
                 if (!tgt) msk = 0;
+                const int eb0 = (int)sizeof(float4) * (first + sb);  // byte offset of bit 0's slot
                 if (BAL == 0) {
-                    const int kb = (int)sizeof(float4) * K;
-                    const int eb0 = (int)sizeof(float4) * (k + sb * K);  // byte offset of bit 0's slot
                     while (msk) {
                         const int ii = __builtin_ctz(msk);
                         msk &= msk - 1;
-                        const int eb = (int)__umul24((unsigned)ii, (unsigned)kb) + eb0;
+                        const int eb = (ii << 4) + eb0;
                         // all of the pair's records read before any is used: one LDS wait per pair
                         // instead of one per record (force pass 3% faster; same arithmetic)
                         const float4 q0 = lds_at(sp[0], eb), q1 = lds_at(sp[1], eb), q3 = lds_at(sp[2], eb);
@@ -1335,7 +1588,7 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
                         force_pair<MHD, ONE_H>(o0, o1, o2, o3, o4, q0, q1, q2, q3, q4, pc, A);
                     }
                 } else {
-                    const int gtot = compact_group(msk, sb, lm, lst);
+                    const int gtot = compact_group(msk, first + sb, lm, lst);
                     __syncthreads();
                     const ListT<CH>* mine = lst + lm.gfirst * 32;  // this target's accepted slots
                     for (int q = k; q < gtot; q += K) {
@@ -1352,8 +1605,8 @@ __device__ __forceinline__ void forces_wave(int vb, const RunDev* __restrict__ r
             }
             __syncthreads();
         }
-        if constexpr (ONE_H) o2 = W.P2[i];
-        force_finish<MHD>(R, W, lm, A, tgt, i, o1, o2, o3, o4, mhd, clean, borve, ch);
+        if constexpr (ONE_H) o2 = s.rec(W.P2);
+        force_finish<MHD>(R, W, lm, A, tgt, s, o1, o2, o3, o4, mhd, clean, borve, ch);
     }
 }
 
@@ -1361,23 +1614,20 @@ template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX = 1, bool GRID
 __global__ __launch_bounds__(64)
 // the balanced loop fits 96 VGPRs without spilling (5 waves per SIMD; the compiler's own choice is 97)
 __attribute__((amdgpu_waves_per_eu(BAL == 1 && !GRID ? 5 : 1)))
-void k_forces(const RunDev* __restrict__ runs, int nruns, int ncell_tot, int nblk_total, StateBuf S, WorkBuf W,
-              int kmax, int balance)
+void k_forces(PairArgs)
 {
     __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[kForcePlanes<MHD, ONE_H && !GRID>][CH];
+    __shared__ float4 sp[kForcePlanes<MHD, ONE_H && !GRID>][kForceSlots<CH>];
     __shared__ ListT<CH> lst[BAL == 1 ? 64 * 32 : 1];  // compaction lists of the balanced pair loop
     __shared__ PreList P;
     if constexpr (GRID) {
         // a persistent grid: each wave walks the supercells at a stride of the grid (a multiple
         // of 8, so every cell a wave visits belongs to its own XCD's range)
-        for (int vb = blockIdx.x; vb < nblk_total; vb += gridDim.x)
-            forces_wave<CH, MIXED, MHD, KT, BAL, RMAX>(vb, runs, nruns, ncell_tot, nblk_total, S, W, kmax, L, sp,
-                                                       lst, P);
+        for (int vb = blockIdx.x; vb < pair_args().nblk_total; vb += gridDim.x)
+            forces_wave<CH, MIXED, MHD, KT, BAL, RMAX>(vb, L, sp, lst, P);
     } else {
         // one supercell per wave
-        forces_wave<CH, MIXED, MHD, KT, BAL, RMAX, ONE_H>((int)blockIdx.x, runs, nruns, ncell_tot, nblk_total, S, W,
-                                                          kmax, L, sp, lst, P);
+        forces_wave<CH, MIXED, MHD, KT, BAL, RMAX, ONE_H>((int)blockIdx.x, L, sp, lst, P);
     }
 }
 
@@ -1421,27 +1671,30 @@ __device__ __forceinline__ uint32_t mask_bits(const uint32_t* row, int lo, int l
 }
 
 template <int CAPD, bool MIXED, bool MHD, int KT>
-__global__ __launch_bounds__(64) void k_density_cell(const RunDev* __restrict__ runs, int nruns, int ncell_tot,
-                                                     int nblk_total, StateBuf S, WorkBuf W, int kmax)
+__global__ __launch_bounds__(64) void k_density_cell(PairArgs)
 {
-    constexpr int RMAX = 1, NS = 27;
+    const PairArgs& args = pair_args();
+    const StateBuf& S = args.S;
+    const WorkBuf& W = args.W;
+    const RunDev* const runs = args.runs;
+    constexpr int RMAX = 1;
     __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[CAPD];
-    const int cell = xcd_cell(blockIdx.x, nblk_total, ncell_tot);
+    __shared__ float4 sp[CAPD + 3];
+    const int cell = xcd_cell(blockIdx.x, args.nblk_total, args.ncell_tot);
     if (cell < 0) return;
     const int t0 = (int)W.cs[cell];
     const int nt = (int)W.cs[cell + 1] - t0;
     if (nt == 0) return;
-    const int r = find_run_by_cell(runs, nruns, cell);
-    const RunDev& R = runs[r];
-    build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L);
-    const int total = L.off[NS];
+    const int r = find_run_by_cell(runs, args.nruns, cell);
+    RunC& R = ((RunC*)runs)[r];
+    int self_v0;
+    const int total = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
     const int lane = threadIdx.x;
-    const LaneMap lm = lane_map(nt, kmax);
+    const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
     const int Lr = (total + K - 1) / K;
     const bool keep = nt <= lm.tpg && Lr <= 32 * kMaskWords && W.nbmask != nullptr;
-    const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
+    const int kern = KT >= 0 ? KT : run_kernel(R.flags);  // compile-time when every run uses one kernel
     const float H2 = R.H2;
     const float gam = R.gamma;
     MaskWriter mw;
@@ -1462,14 +1715,14 @@ __global__ __launch_bounds__(64) void k_density_cell(const RunDev* __restrict__ 
         const float vx = S.vel[0][i], vy = S.vel[1][i], vz = S.vel[2][i];
         const float rho_in = S.rho[i];
         float bx = 0.f, by = 0.f, bz = 0.f, psi = 0.f;
-        if (MHD && R.mhd) {
+        if (MHD && run_mhd(R.flags)) {
             bx = S.B[0][i];
             by = S.B[1][i];
             bz = S.B[2][i];
             psi = S.psi[i];
         }
         const float invh = 1.0f / h;
-        const int self_v = L.off[self_segment<RMAX>(R)] + t;
+        const int self_v = self_v0 + t;
         const int v0 = lm.inwave ? k * Lr : total;
         const int v1 = v0 + Lr < total ? v0 + Lr : total;
         float acc = 0.0f;
@@ -1477,11 +1730,11 @@ __global__ __launch_bounds__(64) void k_density_cell(const RunDev* __restrict__ 
         for (int base = 0; base < total; base += CAPD) {
             const int top = base + CAPD < total ? base + CAPD : total;
             for (int v = base + lane; v < top; v += 64) {
-                const int sg = nb_segment(L, v);
-                float4 p = W.P0[L.start[sg] + (v - L.off[sg])];
-                p.x += L.sh[sg][0];
-                p.y += L.sh[sg][1];
-                p.z += L.sh[sg][2];
+                float4 t4;
+                float4 p = W.P0[list_candidate(L, v, t4)];
+                p.x += t4.x;
+                p.y += t4.y;
+                p.z += t4.z;
                 sp[v - base] = p;
             }
             __syncthreads();
@@ -1489,7 +1742,7 @@ __global__ __launch_bounds__(64) void k_density_cell(const RunDev* __restrict__ 
             const int b = v1 < top ? v1 : top;
             for (int cc = a; cc < b; cc += 32) {
                 const int lim = b - cc < 32 ? b - cc : 32;
-                uint32_t msk = cull32(sp, cc - base, 1, lim, own.x, own.y, own.z, H2);
+                uint32_t msk = cull32(sp + (cc - base), lim, own.x, own.y, own.z, H2);
                 // the self pair passes the cull; its density term is the self term added at the end
                 if (self_v >= cc && self_v < cc + lim) msk &= ~(1u << (self_v - cc));
                 if (!tgt) msk = 0;
@@ -1507,39 +1760,42 @@ __global__ __launch_bounds__(64) void k_density_cell(const RunDev* __restrict__ 
             __syncthreads();
         }
         if (keep) mw.flush();
-        density_finish<MHD>(R, r, S, W, lm, acc, cnt, valid, tgt, spc, live, i, own.w, h, invh, uu, vx, vy, vz,
+        density_finish<MHD>(R, r, S, W, lm, acc, cnt, valid, tgt, spc, live, Slot(t0, (uint32_t)(i - t0)), own.w, h, uu, vx, vy, vz,
                             rho_in, bx, by, bz, psi, gam, kern);
     }
 }
 
 template <int CH, bool MIXED, bool MHD, int KT>
-__global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ runs, int nruns, int ncell_tot,
-                                                    int nblk_total, StateBuf S, WorkBuf W, int kmax)
+__global__ __launch_bounds__(64) void k_forces_cell(PairArgs)
 {
+    const PairArgs& args = pair_args();
+    const StateBuf& S = args.S;
+    const WorkBuf& W = args.W;
+    const RunDev* const runs = args.runs;
     constexpr int NP = MHD ? 5 : 4;
-    constexpr int RMAX = 1, NS = 27;
+    constexpr int RMAX = 1;
     __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[NP][CH];
+    __shared__ float4 sp[NP][CH + 3];
     __shared__ uint16_t lst[kCellListCap];
-    const int cell = xcd_cell(blockIdx.x, nblk_total, ncell_tot);
+    const int cell = xcd_cell(blockIdx.x, args.nblk_total, args.ncell_tot);
     if (cell < 0) return;
     const int t0 = (int)W.cs[cell];
     const int nt = (int)W.cs[cell + 1] - t0;
     if (nt == 0) return;
-    const int r = find_run_by_cell(runs, nruns, cell);
-    const RunDev& R = runs[r];
-    build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L);
-    const int total = L.off[NS];
+    const int r = find_run_by_cell(runs, args.nruns, cell);
+    RunC& R = ((RunC*)runs)[r];
+    int self_v0;
+    const int total = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
     const int lane = threadIdx.x;
-    const LaneMap lm = lane_map(nt, kmax);
+    const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
     const int Lr = (total + K - 1) / K;
     const bool keep = nt <= lm.tpg && Lr <= 32 * kMaskWords;  // the density pass stored masks
-    const int kern = KT >= 0 ? KT : R.kernel;  // compile-time when every run uses one kernel
+    const int kern = KT >= 0 ? KT : run_kernel(R.flags);  // compile-time when every run uses one kernel
     const float H2 = R.H2;
-    const PairConst pc(R, kern, 1.0f, 0.0f);
-    const bool mhd = MHD && R.mhd;
-    const bool clean = mhd && R.cleaning;
+    const PairConst pc(R, kern, R.h0);
+    const bool mhd = MHD && run_mhd(R.flags);
+    const bool clean = mhd && run_cleaning(R.flags);
     const float borve = mhd ? R.borve : 0.0f;
     const float ch = __uint_as_float(W.chbits[r]);
     const uint32_t* mrow = W.nbmask + (size_t)cell * (kMaskWords * 64) + lane;
@@ -1552,7 +1808,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
         const float4 o0 = W.P0[i], o1 = W.P1[i], o2 = W.P2[i], o3 = W.P3[i];
         float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
         if (MHD) o4 = W.P4[i];
-        const int self_v = L.off[self_segment<RMAX>(R)] + t;
+        const int self_v = self_v0 + t;
         const int v0 = lm.inwave ? k * Lr : total;
         const int v1 = v0 + Lr < total ? v0 + Lr : total;
         ForceAcc A = {};
@@ -1583,12 +1839,12 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
             const int top = base + CH < total ? base + CH : total;
             for (int v = base + lane; v < top; v += 64) {
                 const int e = v - base;
-                const int sg = nb_segment(L, v);
-                const int j = L.start[sg] + (v - L.off[sg]);
+                float4 t4;
+                const int j = list_candidate(L, v, t4);
                 float4 p = W.P0[j];
-                p.x += L.sh[sg][0];
-                p.y += L.sh[sg][1];
-                p.z += L.sh[sg][2];
+                p.x += t4.x;
+                p.y += t4.y;
+                p.z += t4.z;
                 sp[0][e] = p;
                 sp[1][e] = W.P1[j];
                 sp[2][e] = W.P2[j];
@@ -1621,7 +1877,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
                     if (keep) {
                         msk = mask_bits(mrow, cc - v0, lim);
                     } else {
-                        msk = cull32(sp[0], cc - base, 1, lim, o0.x, o0.y, o0.z, H2);
+                        msk = cull32(sp[0] + (cc - base), lim, o0.x, o0.y, o0.z, H2);
                         if (self_v >= cc && self_v < cc + lim) msk &= ~(1u << (self_v - cc));
                     }
                     if (!tgt) msk = 0;
@@ -1637,7 +1893,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(const RunDev* __restrict__ r
             }
             __syncthreads();
         }
-        force_finish<MHD>(R, W, lm, A, tgt, i, o1, o2, o3, o4, mhd, clean, borve, ch);
+        force_finish<MHD>(R, W, lm, A, tgt, Slot(t0, (uint32_t)(i - t0)), o1, o2, o3, o4, mhd, clean, borve, ch);
     }
 }
 
@@ -1674,7 +1930,7 @@ __global__ __launch_bounds__(256) void k_kick(const RunDev* __restrict__ runs, S
                 S.vel[2][i] = vz;
                 S.u[i] = u;
             }
-            if (R.mhd) {
+            if (run_mhd(R.flags)) {
                 bx = S.B[0][i];
                 by = S.B[1][i];
                 bz = S.B[2][i];
@@ -1948,6 +2204,11 @@ hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew)
     return hipGetLastError();
 }
 
+static inline PairArgs args_of(const LaunchCtx& c, int nblk)
+{
+    return PairArgs{c.runs, c.nruns, c.ncell_tot, nblk, c.kmax, c.S, c.W};
+}
+
 #define SPH_COMMA ,
 // Instantiate a pair kernel for (precision, MHD fields, smoothing kernel): KT = -1 reads the kernel
 // type per run (batches that mix kernel types).
@@ -1979,44 +2240,38 @@ static void density_ch(const LaunchCtx& c, int nblk)
 {
     const int grid = pair_grid(c, nblk);
     if (grid < nblk)
-        SPH_PAIR_DISPATCH(k_density, grid, CH, SPH_COMMA 1 SPH_COMMA true, c.runs, c.nruns, c.ncell_tot, nblk, c.S,
-                          c.W, c.kmax);
+        SPH_PAIR_DISPATCH(k_density, grid, CH, SPH_COMMA 1 SPH_COMMA true, args_of(c, nblk));
     else
-        SPH_PAIR_DISPATCH(k_density, nblk, CH, , c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W, c.kmax);
+        SPH_PAIR_DISPATCH(k_density, nblk, CH, , args_of(c, nblk));
 }
 
 // supercells finer than H somewhere in the context: the chunked lane loop over the 125-cell stencil
 template <int CH>
 static void density_fine_ch(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_density, nblk, CH, SPH_COMMA 2, c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W, c.kmax);
+    SPH_PAIR_DISPATCH(k_density, nblk, CH, SPH_COMMA 2, args_of(c, nblk));
 }
 
 template <int CAPD>
 static void density_cell_ch(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_density_cell, nblk, CAPD, , c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W, c.kmax);
+    SPH_PAIR_DISPATCH(k_density_cell, nblk, CAPD, , args_of(c, nblk));
 }
 
 template <int CH>
 static void forces_cell_ch(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_forces_cell, nblk, CH, , c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W, c.kmax);
+    SPH_PAIR_DISPATCH(k_forces_cell, nblk, CH, , args_of(c, nblk));
 }
+
+constexpr int kDensitySlots = 256;  // LDS slots of the chunked density pass (DensityLds)
 
 hipError_t launch_density(const LaunchCtx& c)
 {
     const int nblk = nblk_xcd(c.ncell_tot);
-    if (c.rmax == 2) {
-        if (c.density_chunk >= 256) density_fine_ch<256>(c, nblk);
-        else density_fine_ch<128>(c, nblk);
-    } else if (c.balance == 2) {
-        density_cell_ch<512>(c, nblk);
-    } else if (c.density_chunk >= 256) {
-        density_ch<256>(c, nblk);
-    } else {
-        density_ch<128>(c, nblk);
-    }
+    if (c.rmax == 2) density_fine_ch<kDensitySlots>(c, nblk);
+    else if (c.balance == 2) density_cell_ch<512>(c, nblk);
+    else density_ch<kDensitySlots>(c, nblk);
     return hipGetLastError();
 }
 
@@ -2025,21 +2280,18 @@ static void forces_ch(const LaunchCtx& c, int nblk)
 {
     const int grid = pair_grid(c, nblk);
     if (grid < nblk)
-        SPH_PAIR_DISPATCH(k_forces, grid, CH, SPH_COMMA BAL SPH_COMMA 1 SPH_COMMA true, c.runs, c.nruns, c.ncell_tot,
-                          nblk, c.S, c.W, c.kmax, c.balance);
+        SPH_PAIR_DISPATCH(k_forces, grid, CH, SPH_COMMA BAL SPH_COMMA 1 SPH_COMMA true, args_of(c, nblk));
     else if (c.one_h)  // one smoothing length per run: the pair loop neither tests nor averages h
-        SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA BAL SPH_COMMA 1 SPH_COMMA false SPH_COMMA true, c.runs, c.nruns,
-                          c.ncell_tot, nblk, c.S, c.W, c.kmax, c.balance);
+        SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA BAL SPH_COMMA 1 SPH_COMMA false SPH_COMMA true,
+                          args_of(c, nblk));
     else
-        SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA BAL, c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W, c.kmax,
-                          c.balance);
+        SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA BAL, args_of(c, nblk));
 }
 
 template <int CH>
 static void forces_fine_ch(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA 0 SPH_COMMA 2, c.runs, c.nruns, c.ncell_tot, nblk, c.S, c.W,
-                      c.kmax, 0);
+    SPH_PAIR_DISPATCH(k_forces, nblk, CH, SPH_COMMA 0 SPH_COMMA 2, args_of(c, nblk));
 }
 
 hipError_t launch_forces(const LaunchCtx& c)
