@@ -45,14 +45,15 @@ __device__ __forceinline__ int find_run_by_cell(const RunDev* runs, int nruns, i
     return lo;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v)
+// Inclusive sum over the lanes of a wave by DPP row shifts and row broadcasts (six additions).
+__device__ __forceinline__ int dpp_incl_scan(int v)
 {
-    int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        int t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
-    }
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
     return v;
 }
 
@@ -157,42 +158,74 @@ __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ ru
 }
 
 // ------------------------------------------------------------------------------------------------
-// exclusive scan of the per-cell histogram -> cell starts (absolute particle index)
+// exclusive scan of the per-cell histogram -> cell starts (absolute particle index): within blocks of
+// kScanBlock cells in place (k_scan_local), then the blocks' offsets added by k_scatter, which needs the
+// starts first. The offsets of up to kScatterBlocks blocks are scanned by each workgroup of k_scatter for
+// itself (half a million supercells: one load per thread and a scan in LDS, against two more launches of
+// 4.7 us each at any size, and 1.4 us more in the scatter of 2,097,152 particles); more of them are scanned
+// by k_scan_top in between. A table of up to kScatterCells is scanned whole by each workgroup of k_scatter:
+// no other launch, for 0.4 us more in the scatter of 131,044 particles in 5,625 supercells (33 KB of LDS
+// per workgroup bound the limit: four workgroups per compute unit).
 // ------------------------------------------------------------------------------------------------
 constexpr int kScanPerThread = 8;
 constexpr int kScanBlock = 256 * kScanPerThread;
+constexpr int kScatterBlocks = 256;
+constexpr int kScatterCells = 8192;
 
-__global__ __launch_bounds__(256) void k_scan_local(const uint32_t* __restrict__ count, uint32_t* __restrict__ cs,
-                                                    uint32_t* __restrict__ bsum, int n)
+__device__ __forceinline__ uint32_t block_excl_scan256(uint32_t s, uint32_t (&wsum)[4], uint32_t& total)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const uint32_t incl = (uint32_t)dpp_incl_scan((int)s);
+    if (lane == 63) wsum[wid] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        before += w < wid ? wsum[w] : 0u;
+        total += wsum[w];
+    }
+    return before + incl - s;
+}
+
+__global__ __launch_bounds__(256) void k_scan_local(uint32_t* __restrict__ count, uint32_t* __restrict__ bsum, int n)
 {
     __shared__ uint32_t wsum[4];
     const int base = blockIdx.x * kScanBlock + threadIdx.x * kScanPerThread;
     uint32_t v[kScanPerThread];
+    const bool whole = base + kScanPerThread <= n;  // the table is 256-byte aligned: two 16-byte accesses
+    if (whole) {
+        const uint4 a = reinterpret_cast<const uint4*>(count + base)[0];
+        const uint4 b = reinterpret_cast<const uint4*>(count + base)[1];
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanPerThread; ++k) v[k] = base + k < n ? count[base + k] : 0u;
+    }
     uint32_t s = 0;
 #pragma unroll
     for (int k = 0; k < kScanPerThread; ++k) {
-        int e = base + k;
-        v[k] = e < n ? count[e] : 0u;
-        s += v[k];
+        const uint32_t c = v[k];
+        v[k] = s;
+        s += c;
     }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int incl = wave_incl_scan((int)s);
-    if (lane == 63) wsum[wid] = (uint32_t)incl;
-    __syncthreads();
-    uint32_t woff = 0;
-    for (int w = 0; w < wid; ++w) woff += wsum[w];
-    uint32_t run = woff + (uint32_t)incl - s;
+    uint32_t total;
+    const uint32_t off = block_excl_scan256(s, wsum, total);
 #pragma unroll
-    for (int k = 0; k < kScanPerThread; ++k) {
-        int e = base + k;
-        if (e < n) cs[e] = run;
-        run += v[k];
+    for (int k = 0; k < kScanPerThread; ++k) v[k] += off;
+    if (whole) {
+        reinterpret_cast<uint4*>(count + base)[0] = make_uint4(v[0], v[1], v[2], v[3]);
+        reinterpret_cast<uint4*>(count + base)[1] = make_uint4(v[4], v[5], v[6], v[7]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanPerThread; ++k)
+            if (base + k < n) count[base + k] = v[k];
     }
-    if (threadIdx.x == 255) bsum[blockIdx.x] = woff + (uint32_t)incl;
+    if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(1024) void k_scan_top(uint32_t* __restrict__ bsum, int nb, uint32_t* __restrict__ cs,
-                                                   int n)
+// block sums -> exclusive offsets, in place, with the total after the last
+__global__ __launch_bounds__(1024) void k_scan_top(uint32_t* __restrict__ bsum, int nb)
 {
     __shared__ uint32_t wsum[16];
     __shared__ uint32_t carry;
@@ -202,7 +235,7 @@ __global__ __launch_bounds__(1024) void k_scan_top(uint32_t* __restrict__ bsum, 
         int e = base + threadIdx.x;
         uint32_t s = e < nb ? bsum[e] : 0u;
         const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-        int incl = wave_incl_scan((int)s);
+        int incl = dpp_incl_scan((int)s);
         if (lane == 63) wsum[wid] = (uint32_t)incl;
         __syncthreads();
         uint32_t woff = carry;
@@ -212,42 +245,92 @@ __global__ __launch_bounds__(1024) void k_scan_top(uint32_t* __restrict__ bsum, 
         if (threadIdx.x == 1023) carry = woff + (uint32_t)incl;
         __syncthreads();
     }
-    if (threadIdx.x == 0) cs[n] = carry;
-}
-
-__global__ __launch_bounds__(256) void k_scan_add(uint32_t* __restrict__ cs, const uint32_t* __restrict__ bsum, int n)
-{
-    const int base = blockIdx.x * kScanBlock;
-    const uint32_t off = bsum[blockIdx.x];
-    for (int k = threadIdx.x; k < kScanBlock; k += 256) {
-        int e = base + k;
-        if (e < n) cs[e] += off;
-    }
+    if (threadIdx.x == 0) bsum[nb] = carry;
 }
 
 // ------------------------------------------------------------------------------------------------
 // scatter (histogram slot) and gather (final slot = cell start + rank of id within the cell)
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_scatter(const RunDev* __restrict__ runs, StateBuf S, WorkBuf W)
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_scatter(const RunDev* __restrict__ runs, StateBuf S, WorkBuf W, int ncell)
 {
+    __shared__ uint32_t wsum[4];
     const int b = blockIdx.x;
     const RunDev& R = runs[W.blk_run[b]];
     const int64_t local = (int64_t)(b - R.kb_first) * 256 + threadIdx.x;
-    if (local >= R.np) return;
-    const int64_t i = R.p0 + local;
-    const uint32_t slot = W.cs[W.key[i]] + W.rank[i];
-    W.tmp[slot] = (uint32_t)i;
-    W.tmpid[slot] = S.id[i];
+    const bool active = local < R.np;
+    const int64_t i = R.p0 + (active ? local : 0);
+    uint32_t key = 0, rank = 0;
+    uint64_t id = 0;
+    if (active) {
+        key = W.key[i];
+        rank = W.rank[i];
+        id = S.id[i];
+    }
+    const int first = b * 256 + (int)threadIdx.x, step = (int)gridDim.x * 256;  // the entries of cs to write
+    uint32_t slot = 0;
+    if constexpr (WHOLE) {
+        constexpr int kTile = 1024;  // four supercells per thread
+        __shared__ __align__(16) uint32_t start[kScatterCells + 4];
+        uint4 v[kScatterCells / kTile];
+#pragma unroll
+        for (int t = 0; t < kScatterCells / kTile; ++t) {
+            const int e = t * kTile + 4 * (int)threadIdx.x;
+            v[t] = make_uint4(0u, 0u, 0u, 0u);
+            if (e + 4 <= ncell) {
+                v[t] = *reinterpret_cast<const uint4*>(W.count + e);  // the table is 256-byte aligned
+            } else if (e < ncell) {
+                v[t].x = W.count[e];
+                if (e + 1 < ncell) v[t].y = W.count[e + 1];
+                if (e + 2 < ncell) v[t].z = W.count[e + 2];
+            }
+        }
+        uint32_t carry = 0;
+#pragma unroll
+        for (int t = 0; t < kScatterCells / kTile; ++t) {
+            if (t * kTile > ncell) break;  // the entry at ncell is written too
+            uint32_t total;
+            const uint32_t x = carry + block_excl_scan256(v[t].x + v[t].y + v[t].z + v[t].w, wsum, total);
+            *reinterpret_cast<uint4*>(start + t * kTile + 4 * (int)threadIdx.x) =
+                make_uint4(x, x + v[t].x, x + v[t].x + v[t].y, x + v[t].x + v[t].y + v[t].z);
+            carry += total;
+            __syncthreads();
+        }
+        if (ncell == kScatterCells && threadIdx.x == 0) start[ncell] = carry;
+        __syncthreads();
+        slot = start[key] + rank;
+        for (int e = first; e <= ncell; e += step) W.cs[e] = start[e];
+    } else {
+        __shared__ uint32_t pre[kScatterBlocks + 1];  // the scan blocks' offsets, then the total
+        const int nb = (ncell + kScanBlock - 1) / kScanBlock;
+        const uint32_t* off = W.bsum;
+        if (nb <= kScatterBlocks) {
+            uint32_t total;
+            const uint32_t x = block_excl_scan256((int)threadIdx.x < nb ? W.bsum[threadIdx.x] : 0u, wsum, total);
+            pre[threadIdx.x] = x;
+            if ((int)threadIdx.x == nb - 1) pre[nb] = total;
+            __syncthreads();
+            off = pre;
+        }
+        slot = W.count[key] + off[key / kScanBlock] + rank;
+        for (int e = first; e <= ncell; e += step) W.cs[e] = e < ncell ? W.count[e] + off[e / kScanBlock] : off[nb];
+    }
+    if (active) {
+        W.tmp[slot] = (uint32_t)i;
+        W.tmpid[slot] = id;
+    }
 }
 
 template <bool MIXED>
 __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs, StateBuf Sold, StateBuf Snew,
-                                                WorkBuf W, int has_mhd)
+                                                WorkBuf W, int has_mhd, int ncell)
 {
     const int b = blockIdx.x;
     const int r = W.blk_run[b];
     const RunDev& R = runs[r];
     const int64_t local = (int64_t)(b - R.kb_first) * 256 + threadIdx.x;
+    // histogram reset for the next resort
+    for (int e = b * 256 + (int)threadIdx.x; e < ncell; e += (int)gridDim.x * 256) W.count[e] = 0u;
     if (local >= R.np) return;
     const int64_t q = R.p0 + local;
     if (local == 0) W.chbits[r] = 0u;  // cleaning-speed maximum of the coming density pass
@@ -278,7 +361,6 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
     }
     for (; mm < ce; ++mm) rank += (W.tmpid[mm] < myid) ? 1u : 0u;
     const uint32_t f = cb + rank;
-    if (rank == 0) W.count[c] = 0u;  // histogram reset for the next resort
     if (W.perm) W.perm[f] = (int32_t)i;
 
     Snew.id[f] = myid;
@@ -385,18 +467,6 @@ struct Slot {
     }
     __device__ __forceinline__ float4& rec(float4* base) const { return at32(base + t0, t16); }
 };
-
-// Inclusive sum over the lanes of a wave by DPP row shifts and row broadcasts (six additions).
-__device__ __forceinline__ int dpp_incl_scan(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
-}
 
 // Maximum over the wave of values whose bits order as unsigned integers (floats >= +0), as a uniform.
 __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v)
@@ -927,7 +997,7 @@ template <class LT>
 __device__ __forceinline__ int compact_group(uint32_t msk, int first, const LaneMap& m, LT* lst)
 {
     const int na = __popc(msk);
-    const int incl = wave_incl_scan(na);
+    const int incl = dpp_incl_scan(na);
     const int bprev = __shfl(incl, m.gfirst > 0 ? m.gfirst - 1 : 0, 64);
     const int before = m.gfirst > 0 ? bprev : 0;
     const int gtot = __shfl(incl, m.glast, 64) - before;
@@ -1799,7 +1869,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(PairArgs)
 
         // neighbour lists from the stored masks: lane order = candidate order within a target
         const int mine = (keep && tgt) ? mask_count(mrow, 0, v1 - v0) : 0;
-        const int incl = wave_incl_scan(mine);
+        const int incl = dpp_incl_scan(mine);
         const bool listed = keep && __shfl(incl, 63, 64) <= kCellListCap;
         int lo = 0;
         if (listed) {
@@ -1841,7 +1911,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(PairArgs)
                 const int a = v0 > base ? v0 : base;
                 const int b = v1 < top ? v1 : top;
                 const int in_chunk = (tgt && b > a) ? mask_count(mrow, a - v0, b - v0) : 0;
-                const int ci = wave_incl_scan(in_chunk);
+                const int ci = dpp_incl_scan(in_chunk);
                 const int cpre = __shfl(ci, lm.gfirst > 0 ? lm.gfirst - 1 : 0, 64);
                 const int clast = __shfl(ci, lm.glast, 64);
                 const int g = lm.inwave ? clast - (lm.gfirst > 0 ? cpre : 0) : 0;
@@ -2171,20 +2241,23 @@ hipError_t launch_drift_bin(const LaunchCtx& c, double dt_host, int do_drift)
 hipError_t launch_scan(const LaunchCtx& c)
 {
     const int n = c.ncell_tot;
+    if (n <= kScatterCells) return hipSuccess;  // k_scatter scans the histogram itself
     const int nb = (n + kScanBlock - 1) / kScanBlock;
-    k_scan_local<<<nb, 256, 0, c.stream>>>(c.W.count, c.W.cs, c.W.bsum, n);
-    k_scan_top<<<1, 1024, 0, c.stream>>>(c.W.bsum, nb, c.W.cs, n);
-    k_scan_add<<<nb, 256, 0, c.stream>>>(c.W.cs, c.W.bsum, n);
+    k_scan_local<<<nb, 256, 0, c.stream>>>(c.W.count, c.W.bsum, n);
+    if (nb > kScatterBlocks) k_scan_top<<<1, 1024, 0, c.stream>>>(c.W.bsum, nb);
     return hipGetLastError();
 }
 
 hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew)
 {
-    k_scatter<<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W);
-    if (c.mixed)
-        k_gather<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd);
+    if (c.ncell_tot <= kScatterCells)
+        k_scatter<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
     else
-        k_gather<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd);
+        k_scatter<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
+    if (c.mixed)
+        k_gather<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot);
+    else
+        k_gather<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot);
     return hipGetLastError();
 }
 
