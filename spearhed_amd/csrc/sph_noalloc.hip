@@ -107,18 +107,41 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 unsigned char* g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
 
-__global__ void k_set_run(RunDev* dst, RunDev val) { *dst = val; }
+// What a call puts in place before its resort, in one launch (ten launches for the parts took 3.4 us of
+// host time each, 30 of the call's 53 us at 17,550 particles): the run table, the histogram and the run's
+// scalars at zero, ids in input order, a column of zeros and, where the caller has none, the mask and the
+// species (null: the caller's own).
+struct Setup {
+    RunDev run;
+    RunDev* runs;
+    uint32_t* count;
+    int32_t* blk_run;
+    double* dt;
+    uint32_t* chbits;
+    int32_t* prime;
+    float* zero;
+    uint64_t* id;
+    uint8_t* mask;
+    uint8_t* species;
+};
 
-__global__ __launch_bounds__(256) void k_iota64(uint64_t* p, int64_t n)
+__global__ __launch_bounds__(256) void k_setup(Setup P)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = (uint64_t)i;
-}
-
-__global__ __launch_bounds__(256) void k_fill_u8(uint8_t* p, uint8_t v, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
+    if (i == 0) {
+        *P.runs = P.run;
+        *P.dt = 0.0;
+        *P.chbits = 0u;
+        *P.prime = 0;
+    }
+    if (i < P.run.kb_count) P.blk_run[i] = 0;
+    if (i < P.run.ncell) P.count[i] = 0u;  // the histogram starts at zero
+    if (i < P.run.np) {
+        P.zero[i] = 0.0f;
+        P.id[i] = (uint64_t)i;
+        if (P.mask) P.mask[i] = 1;
+        if (P.species) P.species[i] = (uint8_t)SPH_SPECIES_DEFAULT;
+    }
 }
 
 // Sorted slot f came from input index perm[f]: results back into the caller's order.
@@ -285,21 +308,11 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     L.W = W;
     L.stream = s;
 
-    // per-call set-up, all by kernels on the caller's stream (nothing reads host memory later)
-    k_set_run<<<1, 1, 0, s>>>(static_cast<RunDev*>(at(kReg.run)), R);
+    // per-call set-up by a kernel on the caller's stream (nothing reads host memory later)
+    const Setup P{R, static_cast<RunDev*>(at(kReg.run)), W.count, W.blk_run, W.dt, W.chbits, W.prime_flag, zero, A.id,
+                  in->mask ? nullptr : A.mask, in->species ? nullptr : A.species};
+    k_setup<<<grid256(n > R.ncell ? n : R.ncell), 256, 0, s>>>(P);
     e = hipGetLastError();
-    if (e == hipSuccess) e = launch_fill_u32(W.count, 0u, R.ncell, s);  // the histogram starts at zero
-    if (e == hipSuccess) e = launch_fill_u32(reinterpret_cast<uint32_t*>(W.blk_run), 0u, R.kb_count, s);
-    if (e == hipSuccess) e = launch_fill_u32(reinterpret_cast<uint32_t*>(W.dt), 0u, 2, s);
-    if (e == hipSuccess) e = launch_fill_u32(W.chbits, 0u, 1, s);
-    if (e == hipSuccess) e = launch_fill_u32(reinterpret_cast<uint32_t*>(W.prime_flag), 0u, 1, s);
-    if (e == hipSuccess) e = launch_fill_u32(reinterpret_cast<uint32_t*>(zero), 0u, n, s);
-    if (e == hipSuccess) {
-        k_iota64<<<grid256(n), 256, 0, s>>>(A.id, n);
-        if (!in->mask) k_fill_u8<<<grid256(n), 256, 0, s>>>(A.mask, (uint8_t)1, n);
-        if (!in->species) k_fill_u8<<<grid256(n), 256, 0, s>>>(A.species, (uint8_t)SPH_SPECIES_DEFAULT, n);
-        e = hipGetLastError();
-    }
     // the stages of sph_stage_resort + sph_stage_density
     if (e == hipSuccess) e = launch_drift_bin(L, 0.0, 0);
     if (e == hipSuccess) e = launch_scan(L);
