@@ -1071,6 +1071,25 @@ int sph_host_free(void* p)
     return hipHostFree(p) == hipSuccess ? SPH_OK : SPH_E_DEVICE;
 }
 
+// Whether every destination of the table is pinned host memory that kernels reach at the same address (both
+// ends are looked at: a caller may have pinned only the start of an array).
+static bool all_pinned(const CopyTable& t)
+{
+    auto pinned = [](const void* p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();  // ordinary memory: not an error of this call
+            return false;
+        }
+        return a.type == hipMemoryTypeHost && a.devicePointer == p;
+    };
+    for (int i = 0; i < t.n; ++i) {
+        const char* p = static_cast<const char*>(t.col[i].dst);
+        if (!pinned(p) || !pinned(p + t.col[i].bytes - 1)) return false;
+    }
+    return true;
+}
+
 int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conserved* cons)
 {
     if (!c || !d || run < 0 || run >= c->nruns) return SPH_E_INVALID;
@@ -1080,14 +1099,10 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
         return fail(c, SPH_E_INVALID, "download_async: positions need conversion in FP32 contexts; use sph_download");
     const int64_t n = R.np, o = R.p0;
     const StateBuf& S = c->S[c->cur];
-    struct Col {
-        void* dst;
-        const void* src;
-        int64_t bytes;
-    };
-    std::vector<Col> cols;
+    CopyTable cols{};
+    auto push = [&](void* dst, const void* src, int64_t bytes) { cols.col[cols.n++] = {dst, src, bytes}; };
     auto col = [&](void* dst, const void* src, size_t elem) {
-        if (dst && src) cols.push_back({dst, src, (int64_t)elem * n});
+        if (dst && src) push(dst, src, (int64_t)elem * n);
     };
     col(d->id, S.id + o, 8);
     col(d->mask, S.mask + o, 1);
@@ -1115,16 +1130,29 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
     }
     // the FP64 sums and CFL dt that the run's last step (or reduction) left on the device
     static_assert(sizeof(sph_conserved) == 8 * sizeof(double), "sph_conserved is 8 doubles");
-    if (cons) cols.push_back({cons, c->W.cons + (int64_t)run * 8, (int64_t)sizeof(sph_conserved)});
+    if (cons) push(cons, c->W.cons + (int64_t)run * 8, (int64_t)sizeof(sph_conserved));
 
     // Pools snapshot the columns into their device ring on the context's stream (device-to-device,
     // at HBM speed) and copy the snapshot to the host on a second stream, so the copies over PCIe
     // overlap the steps that follow; otherwise, or when the ring is too small for the run, or while
     // the stream is being captured into a graph, the copies go out on the context's stream.
     int64_t need = 0;
-    for (const Col& k : cols) need += (k.bytes + 255) & ~int64_t(255);
+    for (int i = 0; i < cols.n; ++i) need += (cols.col[i].bytes + 255) & ~int64_t(255);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIPTRY(c, hipStreamIsCapturing(c->stream, &cap));
+    // small responses to pinned memory go out by one kernel that writes there
+    const bool direct = cap == hipStreamCaptureStatusNone &&
+                        need <= (c->snap ? kRingCopyBytes : kKernelCopyBytes) && all_pinned(cols);
+    auto copy_out = [&](hipStream_t s) -> int {
+        if (direct) {
+            HIPTRY(c, launch_copy_columns(cols, s));
+            return SPH_OK;
+        }
+        for (int i = 0; i < cols.n; ++i)
+            HIPTRY(c, hipMemcpyAsync(cols.col[i].dst, cols.col[i].src, (size_t)cols.col[i].bytes,
+                                     hipMemcpyDeviceToHost, s));
+        return SPH_OK;
+    };
     int64_t off = 0;
     int rc = SPH_OK;
     if (c->snap && cap == hipStreamCaptureStatusNone && need > 0 && snap_alloc(c, need, off, rc)) {
@@ -1132,18 +1160,17 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
             HIPTRY(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
             HIPTRY(c, hipEventCreateWithFlags(&c->snap_ready, hipEventDisableTiming));
         }
+        CopyTable to_ring = cols;
         int64_t at = off;
-        for (const Col& k : cols) {
-            HIPTRY(c, hipMemcpyAsync(c->snap + at, k.src, (size_t)k.bytes, hipMemcpyDeviceToDevice, c->stream));
-            at += (k.bytes + 255) & ~int64_t(255);
+        for (int i = 0; i < cols.n; ++i) {
+            to_ring.col[i].dst = c->snap + at;
+            cols.col[i].src = c->snap + at;
+            at += (cols.col[i].bytes + 255) & ~int64_t(255);
         }
+        HIPTRY(c, launch_copy_columns(to_ring, c->stream));
         HIPTRY(c, hipEventRecord(c->snap_ready, c->stream));
         HIPTRY(c, hipStreamWaitEvent(c->copy_stream, c->snap_ready, 0));
-        at = off;
-        for (const Col& k : cols) {
-            HIPTRY(c, hipMemcpyAsync(k.dst, c->snap + at, (size_t)k.bytes, hipMemcpyDeviceToHost, c->copy_stream));
-            at += (k.bytes + 255) & ~int64_t(255);
-        }
+        if (int e = copy_out(c->copy_stream)) return e;
         hipEvent_t done = nullptr;
         if (!c->snap_free.empty()) {
             done = c->snap_free.back();
@@ -1156,9 +1183,7 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
         return SPH_OK;
     }
     if (rc) return rc;
-    for (const Col& k : cols)
-        HIPTRY(c, hipMemcpyAsync(k.dst, k.src, (size_t)k.bytes, hipMemcpyDeviceToHost, c->stream));
-    return SPH_OK;
+    return copy_out(c->stream);
 }
 
 int sph_download(sph_ctx* c, int32_t run, sph_host_soa* d)

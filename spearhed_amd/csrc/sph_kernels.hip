@@ -2222,6 +2222,37 @@ static inline int pair_grid(const LaunchCtx& c, int nblk)
     return (c.persistent_waves > 0 && c.persistent_waves < nblk) ? c.persistent_waves : nblk;
 }
 
+// One column per blockIdx.y, copied in the widest units that its addresses allow.
+__global__ __launch_bounds__(256) void k_copy_columns(CopyTable t)
+{
+    char* const dst = static_cast<char*>(t.col[blockIdx.y].dst);
+    const char* const src = static_cast<const char*>(t.col[blockIdx.y].src);
+    const int64_t bytes = t.col[blockIdx.y].bytes;
+    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    auto copy = [&](auto unit) {
+        using T = decltype(unit);
+        const int64_t n = bytes / (int64_t)sizeof(T);
+        for (int64_t i = first; i < n; i += step) reinterpret_cast<T*>(dst)[i] = reinterpret_cast<const T*>(src)[i];
+        const int64_t at = n * (int64_t)sizeof(T) + first;  // fewer than sizeof(T) bytes are left
+        if (at < bytes) dst[at] = src[at];
+    };
+    const uintptr_t low = reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src);
+    if ((low & 15) == 0) copy(uint4{});
+    else if ((low & 7) == 0) copy(uint64_t{});
+    else if ((low & 3) == 0) copy(uint32_t{});
+    else copy(uint8_t{});
+}
+
+hipError_t launch_copy_columns(const CopyTable& t, hipStream_t s)
+{
+    if (t.n <= 0) return hipSuccess;
+    int64_t most = 0;
+    for (int i = 0; i < t.n; ++i) most = most > t.col[i].bytes ? most : t.col[i].bytes;
+    const int64_t blocks = (most + 4095) / 4096;  // 16 bytes per thread
+    k_copy_columns<<<dim3((unsigned)(blocks < 64 ? blocks : 64), (unsigned)t.n), 256, 0, s>>>(t);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;

@@ -30,6 +30,28 @@ struct LaunchCtx {
     hipStream_t stream;
 };
 
+// Columns copied by one launch (launch_copy_columns): any alignment and length >= 1, no overlaps; destinations
+// on the device or in pinned host memory.
+struct CopyTable {
+    struct Col {
+        void* dst;
+        const void* src;
+        int64_t bytes;
+    };
+    int n;
+    Col col[32];  // a response has at most 29 columns and the conserved sums
+};
+// Largest response that a kernel writes to pinned host memory: one launch takes 6 us of host time and 8 us
+// on the stream at 0.28 MB where the copies of 13 columns take 34 and 75. Beyond it the copy engines win
+// when several contexts keep the link busy, since a kernel's writes hold up the other streams' kernels
+// (evaluations of 20^3 / 32^3 / 44^3 / 56^3 / 80^3 particles in turn, 0.35 to 23 MB each: 73 / 79 / 121 /
+// 196 / 459 us by copies, 28 / 55 / 119 / 228 / 634 us by the kernel).
+constexpr int64_t kKernelCopyBytes = int64_t(1) << 21;
+// The same for copies out of a pool's ring, which run beside the next steps on their own stream: 8.9 MB after
+// seven steps of 131,044 particles, 844 us by the kernel, 937 us by copies.
+constexpr int64_t kRingCopyBytes = int64_t(1) << 24;
+
+hipError_t launch_copy_columns(const CopyTable& t, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
 // Copy the state of n_keep runs from A to B: run k's particles [src, src + count) to [dst, dst + count),
 // with (dst, src, count) at tab[3k..3k+2] on the device, dst ascending from 0 and runs contiguous.
