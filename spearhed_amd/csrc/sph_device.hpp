@@ -104,7 +104,8 @@ struct WorkBuf {
     double* partial;  // per kick block: 6 doubles (dt, M, Px, Py, Pz, E)
     double* cons;     // per run: 8 doubles (mass, px, py, pz, energy, dt_next, time, c_h)
     int32_t* blk_run; // per particle-kernel block: run id
-    int32_t* prime_flag; // per run: 1 = the next non-advancing reduction sets the run's first dt
+    int32_t* prime_flag; // per run: 1 = the next non-advancing reduction sets the run's first dt (bit 0; within
+                         // a kick its workgroups count above it)
     int64_t* move_tab;   // per kept run when a pool's run set changes: destination start, source start, count
     int32_t* run_src;    // per run of a new run set: the old run it continues, or -1 for a new run
     double* run_tmp;     // per old run: its dt, time and priming flag, saved while the run set changes
