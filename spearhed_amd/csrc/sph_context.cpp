@@ -440,8 +440,9 @@ int reserve(sph_ctx* c, int64_t cap_p, int64_t cap_c, int cap_r, int cap_kb)
 }
 
 // Upload the run table (and, when given, the block -> run table, the run sources and the move table)
-// through the next staging half, on the context's stream. The host waits only until the copies out
-// of that half from two uploads ago have run.
+// through the next staging half, on the context's stream: one kernel reads them from the pinned half (a copy
+// each took 3.5 us of host time). The host waits only until the kernel that read that half two uploads ago
+// has run.
 int stage_tables(sph_ctx* c, const std::vector<RunDev>& runs, int kb, const std::vector<int32_t>* src,
                  const std::vector<int64_t>* move)
 {
@@ -455,22 +456,24 @@ int stage_tables(sph_ctx* c, const std::vector<RunDev>& runs, int kb, const std:
     int32_t* t_src = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(t_blk) + align256(4 * cap_kb));
     int64_t* t_move = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(t_src) + align256(4 * cap_r));
     const size_t nr = runs.size();
+    CopyTable up{};
+    auto push = [&](void* dst, const void* staged, size_t bytes) { up.col[up.n++] = {dst, staged, (int64_t)bytes}; };
     if (nr > 0) {
         std::copy(runs.begin(), runs.end(), t_runs);
-        HIPTRY(c, hipMemcpyAsync(c->runs_d, t_runs, sizeof(RunDev) * nr, hipMemcpyHostToDevice, c->stream));
+        push(c->runs_d, t_runs, sizeof(RunDev) * nr);
     }
     if (src && nr > 0) {
         for (size_t r = 0; r < nr; ++r)
             for (int b = 0; b < runs[r].kb_count; ++b) t_blk[runs[r].kb_first + b] = (int32_t)r;
-        HIPTRY(c, hipMemcpyAsync(c->W.blk_run, t_blk, sizeof(int32_t) * kb, hipMemcpyHostToDevice, c->stream));
+        push(c->W.blk_run, t_blk, sizeof(int32_t) * kb);
         std::copy(src->begin(), src->end(), t_src);
-        HIPTRY(c, hipMemcpyAsync(c->W.run_src, t_src, sizeof(int32_t) * nr, hipMemcpyHostToDevice, c->stream));
+        push(c->W.run_src, t_src, sizeof(int32_t) * nr);
     }
     if (move && !move->empty()) {
         std::copy(move->begin(), move->end(), t_move);
-        HIPTRY(c, hipMemcpyAsync(c->W.move_tab, t_move, sizeof(int64_t) * move->size(), hipMemcpyHostToDevice,
-                                 c->stream));
+        push(c->W.move_tab, t_move, sizeof(int64_t) * move->size());
     }
+    HIPTRY(c, launch_copy_columns(up, c->stream));
     HIPTRY(c, hipEventRecord(c->stage_ev[h], c->stream));
     return SPH_OK;
 }
@@ -528,8 +531,10 @@ int layout(sph_ctx* c, const std::vector<sph_run_config>& cfg, const std::vector
     c->nkb = kb;
     int rc = stage_tables(c, runs, kb, &src, move);
     if (rc) return rc;
-    HIPTRY(c, launch_remap_runs(c->runs_d, c->W, n_old, nr, c->stream));
-    HIPTRY(c, launch_fill_u32(c->W.count, 0u, c->ncell_cap, c->stream));
+    const bool kept = std::any_of(src.begin(), src.end(), [](int32_t s) { return s >= 0; });
+    HIPTRY(c, launch_remap_runs(c->runs_d, c->W, kept ? n_old : 0, nr, c->stream));
+    // every resort leaves the histogram at zero, so only one that is still to be sorted by is cleared
+    if (c->binned) HIPTRY(c, launch_fill_u32(c->W.count, 0u, c->ncell_cap, c->stream));
     c->binned = false;
     c->sorted = false;
     c->dens_valid = false;
@@ -1046,11 +1051,11 @@ int sph_init_run(sph_ctx* c, int32_t run, const sph_lattice_block* blocks, int32
                 return fail(c, SPH_E_INVALID, "init_run: a block extends outside the run's box");
         }
     const sph_run_config& cfg = c->cfg[run];
-    HIPTRY(c, launch_init_lattice(blocks, n_blocks, R.np, R.p0, seed, jitter, cfg.h0, cfg.gamma, c->mixed ? 1 : 0,
-                                  c->has_mhd ? 1 : 0, c->S[c->cur], c->stream));
     // as an upload: time restarts at 0 and the next step primes the run (enqueued, nothing waits)
+    const RunScalars start{c->W.dt + run, c->W.time + run, c->W.prime_flag + run, R.dt_fixed > 0.0 ? R.dt_fixed : 0.0};
+    HIPTRY(c, launch_init_lattice(blocks, n_blocks, R.np, R.p0, seed, jitter, cfg.h0, cfg.gamma, c->mixed ? 1 : 0,
+                                  c->has_mhd ? 1 : 0, c->S[c->cur], start, c->stream));
     set_one_h(c, run, true);  // the fill gives every particle the run's h0
-    HIPTRY(c, launch_restart_run(c->runs_d, c->W, run, c->stream));
     if (c->binned) HIPTRY(c, launch_fill_u32(c->W.count, 0u, c->ncell_tot, c->stream));
     c->binned = false;
     c->sorted = false;

@@ -68,11 +68,17 @@ struct SetupArgs {
     double jitter;
     float h0, gamma;
     int mixed, has_mhd;
+    RunScalars run;
 };
 
 __global__ __launch_bounds__(256) void k_init_lattice(SetupArgs A, StateBuf S)
 {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g == 0) {
+        *A.run.dt = A.run.dt0;
+        *A.run.time = 0.0;
+        *A.run.prime_flag = 1;
+    }
     if (g >= A.np) return;
     int b = 0;
     while (b + 1 < A.nblocks && g >= A.first[b + 1]) ++b;
@@ -155,7 +161,7 @@ int64_t lattice_sites(const sph_lattice_block* blocks, int n_blocks)
 
 hipError_t launch_init_lattice(const sph_lattice_block* blocks, int n_blocks, int64_t np, int64_t p0, uint64_t seed,
                                double jitter, float h0, float gamma, int mixed, int has_mhd, const StateBuf& S,
-                               hipStream_t stream)
+                               const RunScalars& run, hipStream_t stream)
 {
     SetupArgs A = {};
     int64_t acc = 0;
@@ -176,6 +182,7 @@ hipError_t launch_init_lattice(const sph_lattice_block* blocks, int n_blocks, in
     A.gamma = gamma;
     A.mixed = mixed;
     A.has_mhd = has_mhd;
+    A.run = run;
     if (np <= 0) return hipSuccess;
     k_init_lattice<<<(unsigned)((np + 255) / 256), 256, 0, stream>>>(A, S);
     return hipGetLastError();
