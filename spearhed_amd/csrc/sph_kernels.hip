@@ -533,45 +533,67 @@ __device__ __forceinline__ int self_segment(RunC& R)
     return (side * side * side - 1) / 2;
 }
 
-// Builds the list in LDS; returns its total and sets the list index of the cell's own first particle.
-template <bool MIXED, int RMAX>
-__device__ __forceinline__ int build_nblist(RunC& R, int lcell, const uint32_t* __restrict__ cs,
-                                            NbListR<RMAX>& L, int& self_v0)
+// A load that stays where it is written: the compiler otherwise sinks one below the branches that do not need
+// it, and its latency adds to that of the loads after them.
+__device__ __forceinline__ uint32_t load_early(const uint32_t* p)
 {
-    constexpr int NS = RMAX == 1 ? 27 : 125;
-    const int lane = threadIdx.x;
-    const uint32_t row = div_by((uint32_t)lcell, (uint32_t)R.n[0], R.div[0]);
-    const uint32_t plane = div_by(row, (uint32_t)R.n[1], R.div[1]);
-    const int c[3] = {lcell - (int)row * R.n[0], (int)row - (int)plane * R.n[1], (int)plane};
-    const int side = RMAX == 1 ? 3 : 2 * R.reach + 1;
-    const int nseg = RMAX == 1 ? 27 : side * side * side;
-    int carry = 0;
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// The stencil of a cell: each lane requests the particle ranges of its supercells (the constructor), then the
+// list is built in LDS.
+template <bool MIXED, int RMAX>
+struct Stencil {
+    static constexpr int NS = RMAX == 1 ? 27 : 125, ROUNDS = (NS + 63) / 64;
+    uint32_t st[ROUNDS], end[ROUNDS];
+    float sh[ROUNDS][3];
+    int nseg;
+
+    __device__ __forceinline__ Stencil(RunC& R, int lcell, const uint32_t* __restrict__ cs)
+    {
+        const int n0 = R.n[0], n1 = R.n[1], n2 = R.n[2];
+        const uint32_t div0 = R.div[0], div1 = R.div[1], flags = (uint32_t)R.flags;
+        const int c0 = R.c0;
+        const uint32_t row = div_by((uint32_t)lcell, (uint32_t)n0, div0);
+        const uint32_t plane = div_by(row, (uint32_t)n1, div1);
+        const int c[3] = {lcell - (int)row * n0, (int)row - (int)plane * n1, (int)plane};
+        const int side = RMAX == 1 ? 3 : 2 * R.reach + 1;
+        nseg = RMAX == 1 ? 27 : side * side * side;
 #pragma unroll
-    for (int base = 0; base < NS; base += 64) {
-        const int seg = base + lane;
-        int cnt = 0, st = 0;
-        float sh[3] = {0.f, 0.f, 0.f};
-        if (seg < nseg) {
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int seg = i * 64 + (int)threadIdx.x;
+            st[i] = end[i] = 0;
+            sh[i][0] = sh[i][1] = sh[i][2] = 0.f;
             int cc;
-            if (nb_cell<MIXED, RMAX>(R, c, seg, cc, sh)) {
-                st = (int)cs[cc];
-                cnt = (int)cs[cc + 1] - st;
+            if (seg < nseg && nb_cell<MIXED, RMAX>(R, c, seg, cc, sh[i])) {
+                st[i] = load_early(cs + cc);
+                end[i] = load_early(cs + cc + 1);
             }
         }
-        const int incl = dpp_incl_scan(cnt) + carry;
-        if (seg < NS) {
-            L.t[seg] = make_float4(sh[0], sh[1], sh[2], __int_as_float(st - (incl - cnt)));
-            L.off[seg] = seg < nseg ? incl - cnt : 0;  // past the stencil: overwritten with the total below
-        }
-        if (RMAX == 1) self_v0 = __builtin_amdgcn_readlane(incl - cnt, 13);
-        carry = __builtin_amdgcn_readlane(incl, 63);
     }
-    // the total after the last stencil entry, and in every entry past the run's stencil
-    for (int k = nseg + lane; k <= NS; k += 64) L.off[k] = carry;
-    __syncthreads();
-    if (RMAX != 1) self_v0 = uniform(L.off[self_segment<RMAX>(R)]);
-    return carry;
-}
+    // Builds the list; returns its total and sets the list index of the cell's own first particle.
+    __device__ __forceinline__ int build(RunC& R, NbListR<RMAX>& L, int& self_v0) const
+    {
+        int carry = 0;
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int seg = i * 64 + (int)threadIdx.x;
+            const int cnt = (int)(end[i] - st[i]);
+            const int incl = dpp_incl_scan(cnt) + carry;
+            if (seg < NS) {
+                L.t[seg] = make_float4(sh[i][0], sh[i][1], sh[i][2], __int_as_float((int)st[i] - (incl - cnt)));
+                L.off[seg] = seg < nseg ? incl - cnt : 0;  // past the stencil: overwritten with the total below
+            }
+            if (RMAX == 1) self_v0 = __builtin_amdgcn_readlane(incl - cnt, 13);
+            carry = __builtin_amdgcn_readlane(incl, 63);
+        }
+        // the total after the last stencil entry, and in every entry past the run's stencil
+        for (int k = nseg + (int)threadIdx.x; k <= NS; k += 64) L.off[k] = carry;
+        __syncthreads();
+        if (RMAX != 1) self_v0 = uniform(L.off[self_segment<RMAX>(R)]);
+        return carry;
+    }
+};
 
 // segment of virtual index v (largest k with off[k] <= v, over non-decreasing off[0..NS-1])
 template <int NS>
@@ -1132,7 +1154,7 @@ __device__ __forceinline__ void density_wave(int vb, DensityLds<CH, RMAX>& lds)
     // the targets' box inputs are requested before the neighbour list, so their loads overlap the list's
     const TargetBoxInput box_in = nt <= 64 ? target_box_load(S, W, t0, nt) : TargetBoxInput{};
     int self_v0;
-    const int all = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
+    const int all = Stencil<MIXED, RMAX>(R, cell - R.c0, W.cs).build(R, L, self_v0);
     const int lane = threadIdx.x;
     const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
@@ -1509,27 +1531,26 @@ __device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
     constexpr int NS = RMAX == 1 ? 27 : 125;
     const int cell = xcd_cell(vb, args.nblk_total, args.ncell_tot);
     if (cell < 0) return;
-    const int t0 = uniform((int)W.cs[cell]);
-    const int nt = uniform((int)W.cs[cell + 1]) - t0;
-    if (nt == 0) return;
+    // the supercell's range, the density pass's kept set (stored in its mask row: its count, its first 256
+    // entries and the lane's first 64 mask bits) and the stencil's ranges are all requested before any is
+    // waited for (the kept set is used only if this step's filter and masks apply to the supercell)
+    const int lane = threadIdx.x;
+    const uint32_t first_p = load_early(W.cs + cell), end_p = load_early(W.cs + cell + 1);
+    const uint32_t* row = W.nbmask + (size_t)cell * kRowWords;
+    const uint32_t* const mrow = row + lane;
+    const uint32_t row_last = load_early(row + kRowWords - 1);
+    const uint32_t head0 = load_early(row + kRowWords - 2 - lane), head1 = load_early(row + kRowWords - 66 - lane);
+    const uint32_t mw0 = load_early(mrow), mw1 = load_early(mrow + 64);
     const int r = find_run_by_cell(runs, args.nruns, cell);
     RunC& R = ((RunC*)runs)[r];
-    const int lane = threadIdx.x;
-    // the density pass's kept set, stored in the mask row: its count, its first 256 entries and the lane's
-    // first 64 mask bits are requested before the neighbour list is built, so their loads overlap its
-    // cell-start loads (they are used only if this step's filter and masks apply to the supercell, which
-    // the list decides)
-    const uint32_t* row = W.nbmask + (size_t)cell * kRowWords;
-    uint32_t n_row = kNoList, head[2] = {0, 0};
-    if (nt <= 64) {
-        n_row = row[kRowWords - 1];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) head[q] = row_entries(row, lane + 64 * q);
-    }
-    const uint32_t* const mrow = row + lane;
-    const uint64_t m01 = ((uint64_t)mrow[64] << 32) | mrow[0];
+    const Stencil<MIXED, RMAX> stencil(R, cell - R.c0, W.cs);
+    const int t0 = uniform((int)first_p);
+    const int nt = uniform((int)end_p) - t0;
+    if (nt == 0) return;
+    const uint32_t n_row = nt <= 64 ? row_last : kNoList;
+    const uint64_t m01 = ((uint64_t)mw1 << 32) | mw0;
     int self_v0;
-    const int all = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
+    const int all = stencil.build(R, L, self_v0);
     const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
     // read back where the density pass stored it, else recomputed
@@ -1537,9 +1558,8 @@ __device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
     int total = all;
     const int n_kept = uniform((int)n_row);
     if (pre && (uint32_t)n_kept != kNoList) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            if (2 * (lane + 64 * q) < n_kept) P.v2[lane + 64 * q] = head[q];
+        if (2 * lane < n_kept) P.v2[lane] = (head0 << 16) | (head0 >> 16);
+        if (2 * (lane + 64) < n_kept) P.v2[lane + 64] = (head1 << 16) | (head1 >> 16);
         for (int d = lane + 128; 2 * d < n_kept; d += 64) P.v2[d] = row_entries(row, d);
         __syncthreads();
         total = n_kept;
@@ -1742,7 +1762,7 @@ __global__ __launch_bounds__(64) void k_density_cell(PairArgs)
     const int r = find_run_by_cell(runs, args.nruns, cell);
     RunC& R = ((RunC*)runs)[r];
     int self_v0;
-    const int total = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
+    const int total = Stencil<MIXED, RMAX>(R, cell - R.c0, W.cs).build(R, L, self_v0);
     const int lane = threadIdx.x;
     const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
@@ -1839,7 +1859,7 @@ __global__ __launch_bounds__(64) void k_forces_cell(PairArgs)
     const int r = find_run_by_cell(runs, args.nruns, cell);
     RunC& R = ((RunC*)runs)[r];
     int self_v0;
-    const int total = build_nblist<MIXED, RMAX>(R, cell - R.c0, W.cs, L, self_v0);
+    const int total = Stencil<MIXED, RMAX>(R, cell - R.c0, W.cs).build(R, L, self_v0);
     const int lane = threadIdx.x;
     const LaneMap lm = lane_map(nt, args.kmax);
     const int K = lm.K, k = lm.k;
