@@ -1150,7 +1150,7 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
                         need <= (c->snap ? kRingCopyBytes : kKernelCopyBytes) && all_pinned(cols);
     auto copy_out = [&](hipStream_t s) -> int {
         if (direct) {
-            HIPTRY(c, launch_copy_columns(cols, s));
+            HIPTRY(c, launch_copy_out(cols, s));
             return SPH_OK;
         }
         for (int i = 0; i < cols.n; ++i)

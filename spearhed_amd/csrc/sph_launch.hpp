@@ -41,17 +41,21 @@ struct CopyTable {
     int n;
     Col col[32];  // a response has at most 29 columns and the conserved sums
 };
-// Largest response that a kernel writes to pinned host memory: one launch takes 6 us of host time and 8 us
-// on the stream at 0.28 MB where the copies of 13 columns take 34 and 75. Beyond it the copy engines win
-// when several contexts keep the link busy, since a kernel's writes hold up the other streams' kernels
-// (evaluations of 20^3 / 32^3 / 44^3 / 56^3 / 80^3 particles in turn, 0.35 to 23 MB each: 73 / 79 / 121 /
-// 196 / 459 us by copies, 28 / 55 / 119 / 228 / 634 us by the kernel).
-constexpr int64_t kKernelCopyBytes = int64_t(1) << 21;
+// Largest response that a kernel writes to pinned host memory (launch_copy_out). One launch takes 6 us of host
+// time and 8 us on the stream at 0.28 MB where the copies of 13 columns take 34 and 75. With several contexts
+// keeping the link busy the runtime's copies win beyond it, since a kernel's writes hold up the other streams'
+// kernels (evaluations of 20^3 / 32^3 / 44^3 / 56^3 / 68^3 / 80^3 particles in turn, 0.35 to 23 MB each: 31 /
+// 56 / 122 / 191 / 296 / 464 us by copies, 31 / 55 / 101 / 185 / 290 / 492 us by the kernels; the cubic kernel with
+// two smoothing lengths, 11 MB: 287 by copies, 299).
+constexpr int64_t kKernelCopyBytes = int64_t(8) << 20;
 // The same for copies out of a pool's ring, which run beside the next steps on their own stream: 8.9 MB after
-// seven steps of 131,044 particles, 844 us by the kernel, 937 us by copies.
-constexpr int64_t kRingCopyBytes = int64_t(1) << 24;
+// seven steps of 131,044 particles, 804 us by the kernel, 937 us by copies.
+constexpr int64_t kRingCopyBytes = int64_t(16) << 20;
+// Responses up to this size are written by all XCDs (0.35 MB 31 us a pass instead of 36, 1.4 MB the same).
+constexpr int64_t kWideCopyBytes = int64_t(1) << 20;
 
 hipError_t launch_copy_columns(const CopyTable& t, hipStream_t s);
+hipError_t launch_copy_out(const CopyTable& t, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
 // Copy the state of n_keep runs from A to B: run k's particles [src, src + count) to [dst, dst + count),
 // with (dst, src, count) at tab[3k..3k+2] on the device, dst ascending from 0 and runs contiguous.
