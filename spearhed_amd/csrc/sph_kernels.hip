@@ -89,7 +89,39 @@ __device__ __forceinline__ int xcd_cell(int bid, int nblk_total, int ncell)
 // drift + supercell key + histogram rank (wave-aggregated atomics: particles arrive sorted by
 // cell, so runs of equal keys in a wave take one atomicAdd per run)
 // ------------------------------------------------------------------------------------------------
-template <bool MIXED>
+// A coordinate after a drift of dt, wrapped into a periodic box.
+__device__ __forceinline__ double drifted(const RunDev& R, int a, double x, float v, double dt)
+{
+#pragma clang fp contract(off)
+    x = x + (double)v * dt;
+    if (run_periodic(R.flags, a)) {
+        const double hi = R.lo[a] + R.L[a];
+        if (x >= hi) x = x - R.L[a];
+        else if (x < R.lo[a]) x = x + R.L[a];
+    }
+    return x;
+}
+__device__ __forceinline__ float drifted(const RunDev& R, int a, float x, float v, double dt)
+{
+#pragma clang fp contract(off)
+    x = x + v * (float)dt;
+    if (run_periodic(R.flags, a)) {
+        const float hi = R.lo32[a] + R.L32[a];
+        if (x >= hi) x = x - R.L32[a];
+        else if (x < R.lo32[a]) x = x + R.L32[a];
+    }
+    return x;
+}
+// Whether a particle of run r moves in a drift of dt: a run whose next step primes it (fresh initial data) does
+// not move in that step, nor does a run without a CFL bound (no live target: dt = +inf).
+__device__ __forceinline__ bool moves(int priming, uint8_t species, uint8_t live, double dt)
+{
+    return is_movable(species, live) && !priming && isfinite(dt);
+}
+
+// STORE: the drifted positions are stored; otherwise the gather of the same step drifts them again on their way
+// to their sorted place.
+template <bool MIXED, bool STORE>
 __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ runs, StateBuf S, WorkBuf W,
                                                    double dt_host, int do_drift)
 {
@@ -102,10 +134,7 @@ __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ ru
     uint32_t key = 0xffffffffu;
     if (active) {
         const double dt = dt_host > 0.0 ? dt_host : W.dt[r];
-        const uint8_t live = S.mask[i];
-        // a run whose next step primes it (fresh initial data) does not move in that step, nor does
-        // a run without a CFL bound (no live target: dt = +inf)
-        const bool mov = do_drift && is_movable(S.species[i], live) && !W.prime_flag[r] && isfinite(dt);
+        const bool mov = do_drift && moves(W.prime_flag[r], S.species[i], S.mask[i], dt);
         int c[3];
         for (int a = 0; a < 3; ++a) {
 #pragma clang fp contract(off)
@@ -113,25 +142,15 @@ __global__ __launch_bounds__(256) void k_drift_bin(const RunDev* __restrict__ ru
             if (MIXED) {
                 double x = S.pos64[a][i];
                 if (mov) {
-                    x = x + (double)S.vel[a][i] * dt;
-                    if (run_periodic(R.flags, a)) {
-                        double hi = R.lo[a] + R.L[a];
-                        if (x >= hi) x = x - R.L[a];
-                        else if (x < R.lo[a]) x = x + R.L[a];
-                    }
-                    S.pos64[a][i] = x;
+                    x = drifted(R, a, x, S.vel[a][i], dt);
+                    if (STORE) S.pos64[a][i] = x;
                 }
                 ci = (int)fmin(fmax(floor((x - R.lo[a]) * R.inv_s[a]), 0.0), (double)(R.n[a] - 1));
             } else {
                 float x = S.pos32[a][i];
                 if (mov) {
-                    x = x + S.vel[a][i] * (float)dt;
-                    if (run_periodic(R.flags, a)) {
-                        float hi = R.lo32[a] + R.L32[a];
-                        if (x >= hi) x = x - R.L32[a];
-                        else if (x < R.lo32[a]) x = x + R.L32[a];
-                    }
-                    S.pos32[a][i] = x;
+                    x = drifted(R, a, x, S.vel[a][i], dt);
+                    if (STORE) S.pos32[a][i] = x;
                 }
                 ci = (int)fminf(fmaxf(floorf((x - R.lo32[a]) * R.inv_s32[a]), 0.0f), (float)(R.n[a] - 1));
             }
@@ -323,7 +342,7 @@ __global__ __launch_bounds__(256) void k_scatter(const RunDev* __restrict__ runs
 
 template <bool MIXED>
 __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs, StateBuf Sold, StateBuf Snew,
-                                                WorkBuf W, int has_mhd, int ncell)
+                                                WorkBuf W, int has_mhd, int ncell, double dt_host, int do_drift)
 {
     const int b = blockIdx.x;
     const int r = W.blk_run[b];
@@ -338,6 +357,8 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
     const uint32_t c = W.key[i];
     const uint64_t myid = W.tmpid[q];
     // the particle's old record is read before the rank search, so its loads overlap the search's
+    const double dt = dt_host > 0.0 || !do_drift ? dt_host : W.dt[r];
+    const int priming = do_drift ? W.prime_flag[r] : 0;
     const uint8_t live = Sold.mask[i], sp = Sold.species[i];
     const float m = Sold.mass[i], hh = Sold.h[i], uu = Sold.u[i], rh = Sold.rho[i];
     float vel[3], bf[3] = {0.f, 0.f, 0.f}, ps = 0.f;
@@ -360,6 +381,13 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
         rank += (a0 < myid ? 1u : 0u) + (a1 < myid ? 1u : 0u) + (a2 < myid ? 1u : 0u) + (a3 < myid ? 1u : 0u);
     }
     for (; mm < ce; ++mm) rank += (W.tmpid[mm] < myid) ? 1u : 0u;
+    if (do_drift) {  // the step's drift, binned but not stored
+        if (moves(priming, sp, live, dt))
+            for (int a = 0; a < 3; ++a) {
+                if (MIXED) x64[a] = drifted(R, a, x64[a], vel[a], dt);
+                else x32[a] = drifted(R, a, x32[a], vel[a], dt);
+            }
+    }
     const uint32_t f = cb + rank;
     if (W.perm) W.perm[f] = (int32_t)i;
 
@@ -2379,12 +2407,19 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_drift_bin(const LaunchCtx& c, double dt_host, int do_drift)
+template <bool STORE>
+static void drift_bin(const LaunchCtx& c, double dt_host, int do_drift)
 {
     if (c.mixed)
-        k_drift_bin<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, dt_host, do_drift);
+        k_drift_bin<true, STORE><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, dt_host, do_drift);
     else
-        k_drift_bin<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, dt_host, do_drift);
+        k_drift_bin<false, STORE><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, dt_host, do_drift);
+}
+
+hipError_t launch_drift_bin(const LaunchCtx& c, double dt_host, int do_drift, bool store)
+{
+    if (store) drift_bin<true>(c, dt_host, do_drift);
+    else drift_bin<false>(c, dt_host, do_drift);
     return hipGetLastError();
 }
 
@@ -2398,16 +2433,18 @@ hipError_t launch_scan(const LaunchCtx& c)
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew)
+hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew, double dt_host, int do_drift)
 {
     if (c.ncell_tot <= kScatterCells)
         k_scatter<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
     else
         k_scatter<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
     if (c.mixed)
-        k_gather<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot);
+        k_gather<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
+                                                       do_drift);
     else
-        k_gather<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot);
+        k_gather<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
+                                                       do_drift);
     return hipGetLastError();
 }
 

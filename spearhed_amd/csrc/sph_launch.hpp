@@ -66,9 +66,10 @@ hipError_t launch_remap_runs(const RunDev* runs, const WorkBuf& W, int n_old, in
 hipError_t launch_restart_run(const RunDev* runs, const WorkBuf& W, int run, hipStream_t s);
 hipError_t launch_move_runs(const StateBuf& A, const StateBuf& B, const int64_t* tab, int n_keep, int64_t total,
                             int mixed, int mhd, hipStream_t s);
-hipError_t launch_drift_bin(const LaunchCtx& c, double dt_host, int do_drift);
+// Without store, launch_scatter_gather has to be given the same drift.
+hipError_t launch_drift_bin(const LaunchCtx& c, double dt_host, int do_drift, bool store = true);
 hipError_t launch_scan(const LaunchCtx& c);
-hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew);
+hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew, double dt_host = 0.0, int do_drift = 0);
 hipError_t launch_density(const LaunchCtx& c);
 hipError_t launch_forces(const LaunchCtx& c);
 hipError_t launch_kick(const LaunchCtx& c, double dt_host, int do_kick);
