@@ -340,7 +340,9 @@ __global__ __launch_bounds__(256) void k_scatter(const RunDev* __restrict__ runs
     }
 }
 
-template <bool MIXED>
+// STATE: all of the state is gathered; otherwise only what the density pass of a call without a state needs
+// (identity, mass, h and position: 40 bytes per particle read and written less).
+template <bool MIXED, bool STATE>
 __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs, StateBuf Sold, StateBuf Snew,
                                                 WorkBuf W, int has_mhd, int ncell, double dt_host, int do_drift)
 {
@@ -360,12 +362,12 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
     const double dt = dt_host > 0.0 || !do_drift ? dt_host : W.dt[r];
     const int priming = do_drift ? W.prime_flag[r] : 0;
     const uint8_t live = Sold.mask[i], sp = Sold.species[i];
-    const float m = Sold.mass[i], hh = Sold.h[i], uu = Sold.u[i], rh = Sold.rho[i];
-    float vel[3], bf[3] = {0.f, 0.f, 0.f}, ps = 0.f;
+    const float m = Sold.mass[i], hh = Sold.h[i], uu = STATE ? Sold.u[i] : 0.f, rh = STATE ? Sold.rho[i] : 0.f;
+    float vel[3] = {0.f, 0.f, 0.f}, bf[3] = {0.f, 0.f, 0.f}, ps = 0.f;
     double x64[3] = {0.0, 0.0, 0.0};
     float x32[3] = {0.f, 0.f, 0.f};
     for (int a = 0; a < 3; ++a) {
-        vel[a] = Sold.vel[a][i];
+        if (STATE) vel[a] = Sold.vel[a][i];
         if (MIXED) x64[a] = Sold.pos64[a][i];
         else x32[a] = Sold.pos32[a][i];
     }
@@ -396,14 +398,16 @@ __global__ __launch_bounds__(256) void k_gather(const RunDev* __restrict__ runs,
     Snew.species[f] = sp;
     Snew.mass[f] = m;
     Snew.h[f] = hh;
-    Snew.u[f] = uu;
-    Snew.rho[f] = rh;
+    if (STATE) {
+        Snew.u[f] = uu;
+        Snew.rho[f] = rh;
+    }
     float pc[3];
     const int lc = (int)c - R.c0;
     const int cxyz[3] = {lc % R.n[0], (lc / R.n[0]) % R.n[1], lc / (R.n[0] * R.n[1])};
     for (int a = 0; a < 3; ++a) {
 #pragma clang fp contract(off)
-        Snew.vel[a][f] = vel[a];
+        if (STATE) Snew.vel[a][f] = vel[a];
         if (MIXED) {
             const double x = x64[a];
             Snew.pos64[a][f] = x;
@@ -1117,19 +1121,21 @@ __device__ __forceinline__ void density_finish(RunC& R, int r, const StateBuf& S
         } else {
             rho = rho_in;
         }
-        const float P = (gam - 1.0f) * rho * uu;
-        const float invrho = 1.0f / rho;
-        const float B2 = bx * bx + by * by + bz * bz;
-        const float bdr = invrho * invrho;
-        const float ph = P * bdr;
-        const float pr = (P + 0.5f * B2) * bdr;
-        const float psr = psi * bdr;
-        const float c = sqrtf((gam * P + B2) * invrho);
-        s.rec(W.P1) = make_float4(vx, vy, vz, c);
-        s.rec(W.P2) = make_float4(h, invh, gfac, ph);
-        s.rec(W.P3) = make_float4(pr, 0.5f * rho, bdr, psr);
-        if (MHD) s.rec(W.P4) = make_float4(bx, by, bz, psi);
-        if (tgt) cmax = c;
+        if (MHD || W.P1 != nullptr) {  // null: no force pass follows
+            const float P = (gam - 1.0f) * rho * uu;
+            const float invrho = 1.0f / rho;
+            const float B2 = bx * bx + by * by + bz * bz;
+            const float bdr = invrho * invrho;
+            const float ph = P * bdr;
+            const float pr = (P + 0.5f * B2) * bdr;
+            const float psr = psi * bdr;
+            const float c = sqrtf((gam * P + B2) * invrho);
+            s.rec(W.P1) = make_float4(vx, vy, vz, c);
+            s.rec(W.P2) = make_float4(h, invh, gfac, ph);
+            s.rec(W.P3) = make_float4(pr, 0.5f * rho, bdr, psr);
+            if (MHD) s.rec(W.P4) = make_float4(bx, by, bz, psi);
+            if (tgt) cmax = c;
+        }
     }
     if (writer && valid && !tgt) s.col(W.nnb) = 0;
     if (MHD && run_mhd(R.flags) && run_cleaning(R.flags)) {
@@ -2433,18 +2439,25 @@ hipError_t launch_scan(const LaunchCtx& c)
     return hipGetLastError();
 }
 
+template <bool STATE>
+static void gather(const LaunchCtx& c, const StateBuf& Snew, double dt_host, int do_drift)
+{
+    if (c.mixed)
+        k_gather<true, STATE><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
+                                                           do_drift);
+    else
+        k_gather<false, STATE><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
+                                                            do_drift);
+}
+
 hipError_t launch_scatter_gather(const LaunchCtx& c, const StateBuf& Snew, double dt_host, int do_drift)
 {
     if (c.ncell_tot <= kScatterCells)
         k_scatter<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
     else
         k_scatter<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, c.W, c.ncell_tot);
-    if (c.mixed)
-        k_gather<true><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
-                                                       do_drift);
-    else
-        k_gather<false><<<c.nkb, 256, 0, c.stream>>>(c.runs, c.S, Snew, c.W, c.has_mhd, c.ncell_tot, dt_host,
-                                                       do_drift);
+    if (!c.has_state) gather<false>(c, Snew, dt_host, do_drift);
+    else gather<true>(c, Snew, dt_host, do_drift);
     return hipGetLastError();
 }
 

@@ -14,6 +14,7 @@ struct LaunchCtx {
     int nkb;             // particle-kernel blocks (run-aligned, 256 particles each)
     int mixed;
     int has_mhd;
+    int has_state = 1;  // 0: velocity, u and rho are not part of the state (the resort leaves them alone)
     int density_chunk;
     int force_chunk;
     int kmax;     // max lanes per target in the pair passes

@@ -46,8 +46,8 @@ struct Layout {
 
 struct Regions {
     size_t run, blk, dt, time, chbits, prime, ids, zero, mask1, species0;
-    size_t bid, bmask, bspecies, bpos[3], bvel[3], bmass, bh, bu, brho;
-    size_t nnb, key, rank, tmp, tmpid, count, cs, bsum, p0, p1, p2, p3, perm;
+    size_t bid, bmask, bspecies, bpos[3], bmass, bh, brho;
+    size_t nnb, key, rank, tmp, tmpid, count, cs, bsum, p0, perm;
     size_t total;
 };
 
@@ -71,10 +71,8 @@ constexpr Regions regions()
     g.bmask = l.take(N);
     g.bspecies = l.take(N);
     for (int a = 0; a < 3; ++a) g.bpos[a] = l.take(8 * N);  // FP64 (mixed) or FP32 (plain) positions
-    for (int a = 0; a < 3; ++a) g.bvel[a] = l.take(4 * N);
     g.bmass = l.take(4 * N);
     g.bh = l.take(4 * N);
-    g.bu = l.take(4 * N);
     g.brho = l.take(4 * N);
     g.nnb = l.take(4 * N);
     g.key = l.take(4 * N);
@@ -85,9 +83,6 @@ constexpr Regions regions()
     g.cs = l.take(4 * (C + 1));
     g.bsum = l.take(4 * ((C + 2047) / 2048 + 1));
     g.p0 = l.take(16 * N);
-    g.p1 = l.take(16 * N);
-    g.p2 = l.take(16 * N);
-    g.p3 = l.take(16 * N);
     g.perm = l.take(4 * N);
     g.total = (l.off + 255) & ~size_t(255);
     return g;
@@ -247,12 +242,9 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     for (int a = 0; a < 3; ++a) {
         if (mixed) A.pos64[a] = const_cast<double*>(in->pos[a]);
         else A.pos32[a] = const_cast<float*>(in->pos32[a]);
-        A.vel[a] = zero;
     }
     A.mass = const_cast<float*>(in->mass);
     A.h = const_cast<float*>(in->smoothing_length);
-    A.u = zero;
-    A.rho = zero;
 
     StateBuf B = {};  // the sorted copy
     B.id = static_cast<uint64_t*>(at(kReg.bid));
@@ -261,11 +253,11 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     for (int a = 0; a < 3; ++a) {
         if (mixed) B.pos64[a] = static_cast<double*>(at(kReg.bpos[a]));
         else B.pos32[a] = static_cast<float*>(at(kReg.bpos[a]));
-        B.vel[a] = static_cast<float*>(at(kReg.bvel[a]));
+        B.vel[a] = zero;
     }
     B.mass = static_cast<float*>(at(kReg.bmass));
     B.h = static_cast<float*>(at(kReg.bh));
-    B.u = static_cast<float*>(at(kReg.bu));
+    B.u = zero;
     B.rho = static_cast<float*>(at(kReg.brho));
 
     WorkBuf W = {};
@@ -278,16 +270,14 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     W.cs = static_cast<uint32_t*>(at(kReg.cs));
     W.bsum = static_cast<uint32_t*>(at(kReg.bsum));
     W.P0 = static_cast<float4*>(at(kReg.p0));
-    W.P1 = static_cast<float4*>(at(kReg.p1));
-    W.P2 = static_cast<float4*>(at(kReg.p2));
-    W.P3 = static_cast<float4*>(at(kReg.p3));
     W.dt = static_cast<double*>(at(kReg.dt));
     W.time = static_cast<double*>(at(kReg.time));
     W.chbits = static_cast<uint32_t*>(at(kReg.chbits));
     W.blk_run = static_cast<int32_t*>(at(kReg.blk));
     W.prime_flag = static_cast<int32_t*>(at(kReg.prime));
     W.perm = static_cast<int32_t*>(at(kReg.perm));
-    // nbmask stays null: the density pass keeps no candidate masks (there is no force pass here)
+    // nbmask and P1 to P3 stay null: the density pass keeps no candidate masks and writes no records for a
+    // force pass, which there is none of here
 
     LaunchCtx L{};
     L.runs = static_cast<const RunDev*>(at(kReg.run));
@@ -296,6 +286,7 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     L.nkb = R.kb_count;
     L.mixed = mixed ? 1 : 0;
     L.has_mhd = 0;
+    L.has_state = 0;
     L.density_chunk = 128;  // a context's default tuning
     L.force_chunk = 64;
     L.kmax = 64;
