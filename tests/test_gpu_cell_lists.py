@@ -66,3 +66,18 @@ def test_pair_passes_over_list_sizes(per_cell, variant):
     assert_scaled(g.rho, o.rho[order], o.sc_rho[order], "density")
     for name in ("dvdt", "dudt", "dbdt", "divb", "dpsidt", "vsig"):
         assert np.array_equal(getattr(g, name), getattr(g128, name)), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per_cell", [1, 3, 13, 28, 29])
+def test_mostly_empty_box_gives_the_same_forces(per_cell):
+    """The same particles in a box of 36 times as many supercells of the same edge, nearly all empty: the force
+    pass takes its loads in another order there, and the results keep their bits."""
+    cfg, ps = _case(per_cell, "walls")
+    g = gpu_stages(cfg, ps, "mixed")
+    for a, cells in enumerate((40, 18, 3)):
+        cfg.box_len[a] = cells * 0.25
+    print(f"per_cell {per_cell} in a mostly empty box n={ps.n}", flush=True)
+    w = gpu_stages(cfg, ps, "mixed")
+    for name in ("rho", "nnb", "dvdt", "dudt", "dbdt", "divb", "dpsidt", "vsig"):
+        assert np.array_equal(getattr(g, name), getattr(w, name)), name
