@@ -3,7 +3,7 @@
 A response to pinned memory is written by a kernel up to a size (by all XCDs up to 1 MiB, by one beyond), by
 copies beyond it and to ordinary memory; a pool's goes through its ring. The cases hold one element, column
 lengths that fill no vector, a second run whose columns start off any vector boundary, destinations at such a
-start, and sizes on both sides of the change of kernel and of the limits (8 MiB in a context, 16 MiB out of
+start, and sizes on both sides of the change of kernel and of the limits (12 MiB in a context, 16 MiB out of
 a pool's ring) at 78 bytes per particle.
 """
 from __future__ import annotations
@@ -56,7 +56,7 @@ def _columns(n, ring, shift):
 @pytest.mark.parametrize("pool", [False, True])
 @pytest.mark.parametrize("pinned", [True, False])
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("n", [1, 63, 1001, 13000, 14500, 29001, 105000, 110001, 210000, 220001])
+@pytest.mark.parametrize("n", [1, 63, 1001, 13000, 14500, 29001, 105000, 155000, 170001, 210000, 220001])
 def test_download_async_equals_download(n, shift, pinned, pool):
     runs = [_run(257, 3), _run(n, 4)]
     total = sum(p.n for _, p in runs)
