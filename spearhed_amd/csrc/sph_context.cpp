@@ -15,6 +15,7 @@
 #include "../../include/spearhed_sph.h"
 #include "sph_device.hpp"
 #include "sph_launch.hpp"
+#include "sph_pinned.hpp"
 #include "sph_setup.hpp"
 
 using namespace sph;
@@ -1084,23 +1085,20 @@ int sph_host_free(void* p)
     return hipHostFree(p) == hipSuccess ? SPH_OK : SPH_E_DEVICE;
 }
 
-// Whether every destination of the table is pinned host memory that kernels reach at the same address (both
-// ends are looked at: a caller may have pinned only the start of an array).
-static bool all_pinned(const CopyTable& t)
+// The pinned host allocation around p that kernels reach at the same address, if there is one.
+static PinnedRange pinned_range(const char* p)
 {
-    auto pinned = [](const void* p) {
-        hipPointerAttribute_t a{};
-        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-            (void)hipGetLastError();  // ordinary memory: not an error of this call
-            return false;
-        }
-        return a.type == hipMemoryTypeHost && a.devicePointer == p;
-    };
-    for (int i = 0; i < t.n; ++i) {
-        const char* p = static_cast<const char*>(t.col[i].dst);
-        if (!pinned(p) || !pinned(p + t.col[i].bytes - 1)) return false;
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t start = nullptr;
+    size_t bytes = 0;
+    void* const q = const_cast<char*>(p);
+    const bool ok = hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeHost && a.devicePointer == q &&
+                    hipMemGetAddressRange(&start, &bytes, q) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();  // ordinary memory: not an error of this call
+        return {};
     }
-    return true;
+    return {static_cast<const char*>(start), (int64_t)bytes};
 }
 
 int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conserved* cons)
@@ -1155,7 +1153,8 @@ int sph_download_async(sph_ctx* c, int32_t run, const sph_host_soa* d, sph_conse
     HIPTRY(c, hipStreamIsCapturing(c->stream, &cap));
     // small responses to pinned memory go out by one kernel that writes there
     const bool direct = cap == hipStreamCaptureStatusNone &&
-                        need <= (c->snap ? kRingCopyBytes : kKernelCopyBytes) && all_pinned(cols);
+                        need <= (c->snap ? kRingCopyBytes : kKernelCopyBytes) &&
+                        columns_pinned(cols.col, cols.n, pinned_range);
     auto copy_out = [&](hipStream_t s) -> int {
         if (direct) {
             HIPTRY(c, launch_copy_out(cols, s));
