@@ -2027,21 +2027,20 @@ __global__ __launch_bounds__(64) void k_forces_cell(PairArgs)
 // kick + CFL + FP64 conservation sums (deterministic two-level reduction)
 // ------------------------------------------------------------------------------------------------
 // Reduce a run's kick-block partials in a fixed tree order (one workgroup), publish the conserved sums, set
-// the next dt and advance the time. load(p): the partial at p.
-template <class Load>
+// the next dt and advance the time.
 __device__ __forceinline__ void finalize_run(const RunDev& R, int r, const WorkBuf& W, double dt_host, int advance,
-                                             int priming, const Load& load)
+                                             int priming)
 {
     __shared__ double red[6][4];
     double s[6] = {INFINITY, 0, 0, 0, 0, 0};
-    double* base = W.partial + (int64_t)R.kb_first * 6;
+    const double* base = W.partial + (int64_t)R.kb_first * 6;
     int bb = threadIdx.x;
     for (; bb + 768 < R.kb_count; bb += 1024) {  // four partials per round, loads independent
         double v[4][6];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int q = 0; q < 6; ++q) v[u][q] = load(base + (int64_t)(bb + 256 * u) * 6 + q);
+            for (int q = 0; q < 6; ++q) v[u][q] = base[(int64_t)(bb + 256 * u) * 6 + q];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             s[0] = fmin(s[0], v[u][0]);
@@ -2051,7 +2050,7 @@ __device__ __forceinline__ void finalize_run(const RunDev& R, int r, const WorkB
     for (; bb < R.kb_count; bb += 256) {
         double v[6];
 #pragma unroll
-        for (int q = 0; q < 6; ++q) v[q] = load(base + (int64_t)bb * 6 + q);
+        for (int q = 0; q < 6; ++q) v[q] = base[(int64_t)bb * 6 + q];
         s[0] = fmin(s[0], v[0]);
 #pragma unroll
         for (int q = 1; q < 6; ++q) s[q] += v[q];
@@ -2096,10 +2095,12 @@ __device__ __forceinline__ void finalize_run(const RunDev& R, int r, const WorkB
     }
 }
 
-// Up to this many workgroups in all, the kick finalises its runs itself, one launch less: 4,096 particles
-// 7.6 us instead of 5.4 + 4.1, 32,832 8.5 instead of 5.5 + 4.5. At 512 workgroups their counting off on one
-// word makes it 15.0 instead of 7.7 + 4.7.
-constexpr int kKickFinalizes = 256;
+// Up to this many workgroups in all, the kick finalises its runs itself, one launch less. Each workgroup's
+// release writes its XCD's L2 back, so the kick grows with their number: 16 workgroups 7.9 us against 5.6 of the
+// kick and 4.5 of the finalising launch, 62 8.0 against 5.6 + 4.7, 128 8.8 against 5.7 + 4.7, 250 12.2 against
+// 6.3 + 4.7. A step alone takes 64.1 us against 64.8 with 16, 66.5 against 67.4 with 62, as long either way with
+// 128 and 0.5 us longer with 168; contexts in turn with 129 take 1.4% longer a pass.
+constexpr int kKickFinalizes = 64;
 
 // LAST: the last workgroup of a run to come here also finalises the run.
 template <bool MIXED, bool LAST>
@@ -2110,7 +2111,9 @@ __global__ __launch_bounds__(256) void k_kick(const RunDev* __restrict__ runs, S
     const int b = blockIdx.x;
     const int r = W.blk_run[b];
     const RunDev& R = runs[r];
-    const int priming = W.prime_flag[r] & 1;  // bit 0; the workgroups count themselves off above it (LAST)
+    // bit 0; the workgroups count themselves off above it (LAST), so the load is atomic as the count is
+    const int priming =
+        LAST ? __hip_atomic_load(&W.prime_flag[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 1 : W.prime_flag[r];
     const int64_t local = (int64_t)(b - R.kb_first) * 256 + threadIdx.x;
     double v_dt = INFINITY, v_m = 0, v_px = 0, v_py = 0, v_pz = 0, v_e = 0;
     if (local < R.np) {
@@ -2193,31 +2196,21 @@ __global__ __launch_bounds__(256) void k_kick(const RunDev* __restrict__ runs, S
         double s;
         if (q == 0) s = fmin(fmin(red[0][0], red[0][1]), fmin(red[0][2], red[0][3]));
         else s = (red[q][0] + red[q][1]) + (red[q][2] + red[q][3]);
-        double* const p = W.partial + (int64_t)b * 6 + q;
-        if constexpr (LAST) {
-            // The partials cross the XCDs' caches within this kernel, so they are written and read by
-            // read-modify-writes at agent scope, like the histogram; a write has happened once its old value
-            // is here, and only then does the workgroup count itself off.
-            const uint64_t old = __hip_atomic_exchange(reinterpret_cast<unsigned long long*>(p),
-                                                       (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("" ::"v"(old) : "memory");
-        } else {
-            *p = s;
-        }
+        W.partial[(int64_t)b * 6 + q] = s;
     }
     if constexpr (LAST) {
+        // The partials pass between workgroups, and XCDs with an L2 each, within this kernel: the workgroup's are
+        // stored before the barrier, its count-off releases them, and the last one acquires everybody's after its
+        // own count-off and before the barrier that its loads come after.
         __shared__ int last;
-        if (threadIdx.x == 0) {  // the wave that wrote the partials
-            const int before = __hip_atomic_fetch_add(&W.prime_flag[r], 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int before = __hip_atomic_fetch_add(&W.prime_flag[r], 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
             last = (before >> 1) == R.kb_count - 1;
+            if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
         __syncthreads();
-        if (last)
-            finalize_run(R, r, W, dt_host, do_kick, priming, [](double* p) {
-                return __longlong_as_double((long long)__hip_atomic_fetch_or(
-                    reinterpret_cast<unsigned long long*>(p), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            });
+        if (last) finalize_run(R, r, W, dt_host, do_kick, priming);
     }
 }
 
@@ -2226,7 +2219,7 @@ __global__ __launch_bounds__(256) void k_finalize(const RunDev* __restrict__ run
                                                   int advance)
 {
     const int r = blockIdx.x;
-    finalize_run(runs[r], r, W, dt_host, advance, W.prime_flag[r], [](const double* p) { return *p; });
+    finalize_run(runs[r], r, W, dt_host, advance, W.prime_flag[r]);
 }
 
 
