@@ -661,12 +661,14 @@ __device__ __forceinline__ int nb_segment(const NbListT<NS>& L, int v)
 // ------------------------------------------------------------------------------------------------
 constexpr int kPreCap = 768;  // larger stencils, and supercells of more than 64 particles, stage whole
 
+constexpr uint16_t kNoSelf = 0xffff;  // past every staged slot
+
 struct PreList {
     union {
         uint16_t v[kPreCap];       // the kept candidates in list order (pre_entry)
         uint32_t v2[kPreCap / 2];  // the same, two entries per word
     };
-    uint16_t self_s[64];  // kept index of each target of the supercell (a target is always kept)
+    uint16_t self_s[64];  // kept index of each target of the supercell; kNoSelf of one at no finite position
     uint32_t seg4[64];    // see fill_segments
 };
 
@@ -812,6 +814,8 @@ __device__ __forceinline__ int prefilter(const NbListT<NS>& L, const WorkBuf& W,
     // monotone), and both sums of squares round in the same fma order, so the cull's r2 is never
     // below this d2. The 2^-13 margin on H^2 is kept on top of that.
     const float H2m = B.lx <= B.hx ? H2 * (1.0f + 1.0f / 8192.0f) : -1.0f;  // no targets: nothing is kept
+    // a target is kept, unless its position is not finite: its distance to the box is not a number then
+    self_s[lane] = kNoSelf;
     int count = 0;
     int seg_off = 0, seg_cnt = 0;  // lane's own segment of the 27
     uint32_t last = 0;
@@ -865,7 +869,8 @@ __device__ __forceinline__ int prefilter(const NbListT<NS>& L, const WorkBuf& W,
 }
 
 // Cull lim (<= 32) consecutive lane candidates in the LDS slots from sp on: bit ii set iff r2 < H2, read
-// off the sign of r2 - H2 (exact: the rounded difference has the sign of the exact one). Returns
+// off the sign of |r2| - H2 (exact: the rounded difference has the sign of the exact one; r2 that is not a
+// number, a position not being finite, loses the sign that it may have: never a neighbour). Returns
 // LSB-first bits. Candidates go four at a time, all four LDS reads issued before any is used, up to
 // three slots past lim (the caller's LDS array has them; their bits are cut off).
 __device__ __forceinline__ uint32_t cull32(const float4* __restrict__ sp, int lim, float xi, float yi, float zi,
@@ -878,13 +883,13 @@ __device__ __forceinline__ uint32_t cull32(const float4* __restrict__ sp, int li
         __builtin_amdgcn_sched_barrier(0);
         float dx, dy, dz;
         const float r2a = geom_r2(xi, yi, zi, q0, dx, dy, dz);
-        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2a - H2), 31);  // (m << 1) | sign
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(fabsf(r2a) - H2), 31);  // (m << 1) | sign
         const float r2b = geom_r2(xi, yi, zi, q1, dx, dy, dz);
-        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2b - H2), 31);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(fabsf(r2b) - H2), 31);
         const float r2c = geom_r2(xi, yi, zi, q2, dx, dy, dz);
-        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2c - H2), 31);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(fabsf(r2c) - H2), 31);
         const float r2d = geom_r2(xi, yi, zi, q3, dx, dy, dz);
-        m = __builtin_amdgcn_alignbit(m, __float_as_uint(r2d - H2), 31);
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(fabsf(r2d) - H2), 31);
     }
     const uint32_t bits = __builtin_bitreverse32(m) >> (32 - n);
     return lim == 32 ? bits : bits & ((1u << lim) - 1u);
