@@ -1371,9 +1371,9 @@ struct PairConst {
 // ONE_H: every particle of the run has the same smoothing length, so record 2 of the neighbour is not
 // read; the same bits as the general form. The pass is bound by VALU issue, so the pair is a straight
 // run of 72 instructions (three transcendental) with no branch or select in it: the support test is the
-// clamp of kslope, the r > 0 guard a lower bound on r2 (coincident particles then have r = 0, a finite
-// 1/r and exact zeros in every term), runs without viscosity or cleaning take zeros through the same
-// code, and the exact halves and doublings of the viscosity are folded away (rho / 2 in the record:
+// clamp of kslope, the r > 0 guard a lower bound on r2 (every normal r2 is itself; coincident particles have
+// r = 0, a finite 1/r and exact zeros in every term), runs without viscosity or cleaning take zeros through
+// the same code, and the exact halves and doublings of the viscosity are folded away (rho / 2 in the record:
 // 1 / (rho_i/2 + rho_j/2) is the mean density's reciprocal). Every product and fused multiply-add is
 // written out, contraction off, so all instantiations round alike. Against the branched form with five
 // staged records (85 instructions) the force pass took 0.75 -> 0.69 ms at 2,097,152 particles.
@@ -1385,7 +1385,7 @@ __device__ __forceinline__ void force_pair(const float4& o0, const float4& o1, c
 #pragma clang fp contract(off)
     float dx, dy, dz;
     const float r2 = geom_r2(o0.x, o0.y, o0.z, q0, dx, dy, dz);
-    const float invR = fast_rsq(fmaxf(r2, 1e-37f));
+    const float invR = fast_rsq(fmaxf(r2, 0x1p-126f));  // the least normal number: v_rsq_f32 gives inf below it
     const float rr = r2 * invR;
     const float ms_i = q0.w * kslope(C.kern, invR, rr * (ONE_H ? C.invh : o2.y), ONE_H ? C.gfac : o2.z);
     float ms_j = ms_i;
