@@ -669,7 +669,6 @@ struct PreList {
         uint32_t v2[kPreCap / 2];  // the same, two entries per word
     };
     uint16_t self_s[64];  // kept index of each target of the supercell; kNoSelf of one at no finite position
-    uint32_t seg4[64];    // see fill_segments
 };
 
 // A kept-list entry: the list index (< kPreCap <= 1024) and, for the 27-cell stencil, its segment, so that
@@ -1563,13 +1562,21 @@ __device__ __forceinline__ void force_finish(RunC& R, const WorkBuf& W, const La
 template <bool MHD, bool ONE_H>
 constexpr int kForcePlanes = 3 + (MHD ? 1 : 0) + (ONE_H ? 0 : 1);
 
-// LDS slots of a force chunk: CH, the odd-stride rounding of ChunkMap and the cull's three.
-template <int CH>
-constexpr int kForceSlots = CH + 8;
+// LDS slots of a force chunk in each of NP planes: CH and some more for the odd-stride rounding of ChunkMap and
+// for the cull's three. With five planes only four more, and the cull reads on into the second plane: the LDS
+// then stays within 7,680 bytes (64 slots, MHD, unequal h), 21 waves per compute unit, for which the compiler
+// keeps to 96 registers, 5 waves per SIMD. With eight more and the filter's segment table beside them (it lies in
+// the slots while the filter runs) it was 8,224 bytes and 98 registers, 4 waves: the cubic force pass of 262,144
+// particles took 102.5 us instead of 98.2, the quintic 112.3 instead of 107.9, the Wendland 96.0 instead of 93.3.
+template <int CH, int NP>
+constexpr int kForceSlots = CH + (NP == 5 ? 4 : 8);
+template <int CH, int NP>
+constexpr int kForceCap = kForceSlots<CH, NP> + (NP == 5 ? 3 : 0);  // ChunkMap's CAP
 
-template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX, bool ONE_H = false>
+template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX, bool ONE_H = false,
+          int NP = kForcePlanes<MHD, ONE_H>>
 __device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
-                                            float4 (&sp)[kForcePlanes<MHD, ONE_H>][kForceSlots<CH>],
+                                            float4 (&sp)[NP][kForceSlots<CH, NP>],
                                             ListT<CH> (&lst)[BAL == 1 ? 64 * 32 : 1], PreList& P)
 {
     const PairArgs& args = pair_args();
@@ -1622,10 +1629,10 @@ __device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
         total = n_kept;
     } else if (pre) {
         total = prefilter<NS>(L, W, target_box(target_box_load(S, W, t0, nt), nt), nt, all, self_v0, R.H2, P.v,
-                              P.self_s, P.seg4);
+                              P.self_s, reinterpret_cast<uint32_t*>(sp[0]));
     }
     const StageOrder so(total);  // the density pass's staged order: its masks replay slot by slot
-    const ChunkMap cm(kForceSlots<CH>, lm);
+    const ChunkMap cm(kForceCap<CH, NP>, lm);
     const int per_lane = uquot(total + K - 1, K, lm.rK);
     const int kern = KT >= 0 ? KT : run_kernel(R.flags);  // compile-time when every run uses one kernel
     const float H2 = R.H2;
@@ -1741,14 +1748,19 @@ __device__ __forceinline__ void forces_wave(int vb, NbListR<RMAX>& L,
     }
 }
 
+// The default pass over MHD fields and unequal h takes 98 registers, 4 waves per SIMD, unless it is held to 96.
+// The balanced loop is held too; its LDS leaves it 4 waves with unequal h, and it takes 100 there.
+template <int CH, bool MHD, int BAL, int RMAX, bool GRID, bool ONE_H>
+constexpr int kForceWaves = !GRID && (BAL == 1 || (CH == 64 && MHD && !ONE_H && RMAX == 1)) ? 5 : 1;
+
 template <int CH, bool MIXED, bool MHD, int KT, int BAL, int RMAX = 1, bool GRID = false, bool ONE_H = false>
 __global__ __launch_bounds__(64)
-// the balanced loop fits 96 VGPRs without spilling (5 waves per SIMD; the compiler's own choice is 97)
-__attribute__((amdgpu_waves_per_eu(BAL == 1 && !GRID ? 5 : 1)))
+__attribute__((amdgpu_waves_per_eu(kForceWaves<CH, MHD, BAL, RMAX, GRID, ONE_H>)))
 void k_forces(PairArgs)
 {
     __shared__ NbListR<RMAX> L;
-    __shared__ float4 sp[kForcePlanes<MHD, ONE_H && !GRID>][kForceSlots<CH>];
+    constexpr int NP = kForcePlanes<MHD, ONE_H && !GRID>;
+    __shared__ float4 sp[NP][kForceSlots<CH, NP>];
     __shared__ ListT<CH> lst[BAL == 1 ? 64 * 32 : 1];  // compaction lists of the balanced pair loop
     __shared__ PreList P;
     if constexpr (GRID) {
