@@ -280,7 +280,6 @@ LaunchCtx lctx(sph_ctx* c)
     L.nkb = c->nkb;
     L.mixed = c->mixed ? 1 : 0;
     L.has_mhd = c->has_mhd ? 1 : 0;
-    L.density_chunk = c->tune.density_chunk;
     L.kmax = std::max(1, std::min(64, c->tune.max_lanes_per_target));
     L.S = c->S[c->cur];
     L.force_chunk = c->tune.force_chunk;

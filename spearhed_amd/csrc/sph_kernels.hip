@@ -2524,27 +2524,27 @@ static inline PairArgs args_of(const LaunchCtx& c, int nblk)
         }                                                                                           \
     } while (0)
 
-template <int CH>
-static void density_ch(const LaunchCtx& c, int nblk)
+constexpr int kDensitySlots = 256;      // LDS slots of the chunked density pass (DensityLds)
+constexpr int kDensityCellSlots = 512;  // and of the whole-cell one
+
+static void density_chunked(const LaunchCtx& c, int nblk)
 {
     const int grid = pair_grid(c, nblk);
     if (grid < nblk)
-        SPH_PAIR_DISPATCH(k_density, grid, CH, SPH_COMMA 1 SPH_COMMA true, args_of(c, nblk));
+        SPH_PAIR_DISPATCH(k_density, grid, kDensitySlots, SPH_COMMA 1 SPH_COMMA true, args_of(c, nblk));
     else
-        SPH_PAIR_DISPATCH(k_density, nblk, CH, , args_of(c, nblk));
+        SPH_PAIR_DISPATCH(k_density, nblk, kDensitySlots, , args_of(c, nblk));
 }
 
 // supercells finer than H somewhere in the context: the chunked lane loop over the 125-cell stencil
-template <int CH>
-static void density_fine_ch(const LaunchCtx& c, int nblk)
+static void density_fine(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_density, nblk, CH, SPH_COMMA 2, args_of(c, nblk));
+    SPH_PAIR_DISPATCH(k_density, nblk, kDensitySlots, SPH_COMMA 2, args_of(c, nblk));
 }
 
-template <int CAPD>
-static void density_cell_ch(const LaunchCtx& c, int nblk)
+static void density_cell(const LaunchCtx& c, int nblk)
 {
-    SPH_PAIR_DISPATCH(k_density_cell, nblk, CAPD, , args_of(c, nblk));
+    SPH_PAIR_DISPATCH(k_density_cell, nblk, kDensityCellSlots, , args_of(c, nblk));
 }
 
 template <int CH>
@@ -2553,14 +2553,12 @@ static void forces_cell_ch(const LaunchCtx& c, int nblk)
     SPH_PAIR_DISPATCH(k_forces_cell, nblk, CH, , args_of(c, nblk));
 }
 
-constexpr int kDensitySlots = 256;  // LDS slots of the chunked density pass (DensityLds)
-
 hipError_t launch_density(const LaunchCtx& c)
 {
     const int nblk = nblk_xcd(c.ncell_tot);
-    if (c.rmax == 2) density_fine_ch<kDensitySlots>(c, nblk);
-    else if (c.balance == 2) density_cell_ch<512>(c, nblk);
-    else density_ch<kDensitySlots>(c, nblk);
+    if (c.rmax == 2) density_fine(c, nblk);
+    else if (c.balance == 2) density_cell(c, nblk);
+    else density_chunked(c, nblk);
     return hipGetLastError();
 }
 

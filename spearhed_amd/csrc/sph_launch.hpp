@@ -15,7 +15,6 @@ struct LaunchCtx {
     int mixed;
     int has_mhd;
     int has_state = 1;  // 0: velocity, u and rho are not part of the state (the resort leaves them alone)
-    int density_chunk;
     int force_chunk;
     int kmax;     // max lanes per target in the pair passes
     int balance;  // pair_balance: 1 = the force pass shares a target's accepted pairs among its K lanes,

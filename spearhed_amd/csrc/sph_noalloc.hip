@@ -287,8 +287,7 @@ extern "C" int sph_density_noalloc(const sph_run_config* cfg, int32_t precision,
     L.mixed = mixed ? 1 : 0;
     L.has_mhd = 0;
     L.has_state = 0;
-    L.density_chunk = 128;  // a context's default tuning
-    L.force_chunk = 64;
+    L.force_chunk = 64;  // a context's default tuning
     L.kmax = 64;
     L.balance = 0;
     L.kern = cfg->kernel;
