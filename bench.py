@@ -317,7 +317,7 @@ def main():
     ap.add_argument("--precision", default="mixed", choices=["mixed", "fp32"])
     ap.add_argument("--tune", action="store_true", help="run the autotuner before timing")
     ap.add_argument("--tuning", default="", help="JSON launch shape for the main workload, e.g. "
-                    "'{\"pair_balance\": 2, \"density_chunk\": 512, \"force_chunk\": 256}'")
+                    "'{\"pair_balance\": 2, \"density_chunk\": 512, \"force_chunk\": 128}'")
     ap.add_argument("--cell-factor", type=float, default=0.0,
                     help="supercell edge in interaction radii for the main workload (0: the default, 1; 0.5: the "
                          "125-supercell stencil)")

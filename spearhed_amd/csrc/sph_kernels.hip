@@ -1,13 +1,15 @@
 // sph_kernels.hip -- hand-written gfx950 kernels of the SPH-MHD particle step.
 //
 // Stage -> kernels (reference stage in brackets):
-//   drift + bin   k_drift_bin        [PushVelocity, PushVelocity.hpp:35-42; + supercell key/histogram]
-//   resort        k_scan_local/top/add, k_scatter, k_gather
+//   drift + bin   k_drift_bin        [PushVelocity, PushVelocity.hpp:35-42; + supercell key/histogram; large
+//                                     steps store the drift in k_gather]
+//   resort        k_scan_local, k_scan_top (large tables), k_scatter, k_gather
 //                                    [UpdateVolumes RegionBoundsUpdate.hpp:175-214 and the frame index
 //                                     FrameIndex.hpp:209-296, replaced by a counting sort by (cell, id)]
 //   density       k_density<CH>      [UpdateDensity, DensitySummation.hpp:104-138]
 //   forces        k_forces<CH, MHD>  [UpdateHydroForces, HydroForces.hpp:183-214, + AV/MHD/cleaning]
-//   integrate     k_kick, k_finalize [EulerIntegrate, EulerIntegrate.hpp:43-52, + CFL and FP64 sums]
+//   integrate     k_kick, k_finalize (within k_kick for small sets)
+//                                    [EulerIntegrate, EulerIntegrate.hpp:43-52, + CFL and FP64 sums]
 //
 // Pair passes: one wave64 per target supercell. The 27 neighbour supercells form a virtual list
 // whose candidates within the support radius of the targets' bounding box are staged chunk by
@@ -1369,7 +1371,7 @@ struct PairConst {
 // 2 (h, 1/h, gfac, ph), 3 (pr, rho / 2, bdr, psr), 4 (B, psi).
 // ONE_H: every particle of the run has the same smoothing length, so record 2 of the neighbour is not
 // read; the same bits as the general form. The pass is bound by VALU issue, so the pair is a straight
-// run of 72 instructions (three transcendental) with no branch or select in it: the support test is the
+// run of 72 instructions (three transcendental; 77 with the loop's own) with no branch or select in it: the support test is the
 // clamp of kslope, the r > 0 guard a lower bound on r2 (every normal r2 is itself; coincident particles have
 // r = 0, a finite 1/r and exact zeros in every term), runs without viscosity or cleaning take zeros through
 // the same code, and the exact halves and doublings of the viscosity are folded away (rho / 2 in the record:
@@ -1487,8 +1489,8 @@ __device__ __forceinline__ float row_shr(float x)
 // K partial force sums of a target combined (deterministic), field by field; then one lane per
 // target writes its derivatives, signal speed and div B. For K = 2, 4, 8 or 16 a target's lanes lie
 // in one 16-lane row, and log2 K DPP steps (each lane adds the partial of the lane 1, 2, 4, ... below
-// it) leave the target's total in its last lane; other K take the shuffles of each lane's partial
-// in lane order to every lane of the target.
+// it) leave the target's total in its last lane; other K take K - 1 wave shifts by one lane, which add
+// the partials in lane order and leave the total there too.
 template <bool MHD>
 __device__ __forceinline__ void force_finish(RunC& R, const WorkBuf& W, const LaneMap& lm, ForceAcc& A, bool tgt,
                                              const Slot& s, const float4& o1, const float4& o2, const float4& o3,

@@ -46,7 +46,7 @@ struct CopyTable {
 // keeping the link busy the runtime's copies win beyond it, since a kernel's writes hold up the other streams'
 // kernels (evaluations of 20^3 / 32^3 / 44^3 / 56^3 / 62^3 / 70^3 / 80^3 particles in turn, 0.35 to 23 MB each: 31 /
 // 56 / 122 / 191 / 260 / 325 / 464 us by copies, 31 / 55 / 101 / 185 / 235 / 334 / 492 us by the kernels; 13.2 MB
-// beside the cubic kernel 267 to 308 by copies, 297 by the kernels).
+// beside the cubic kernel 260 to 299 by copies, 297 by the kernels).
 constexpr int64_t kKernelCopyBytes = int64_t(12) << 20;
 // The same for copies out of a pool's ring, which run beside the next steps on their own stream: 8.9 MB after
 // seven steps of 131,044 particles, 804 us by the kernel, 937 us by copies.

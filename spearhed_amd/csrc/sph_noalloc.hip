@@ -4,13 +4,13 @@
 // run whose particles the caller holds in device columns, and writes density and neighbour counts
 // in the caller's particle order.
 //
-// All working memory (run table, sorted copy of the particles, supercell histogram and starts,
-// interaction records, permutation) lives in `scratch`, one file-scope device array per GPU that
+// All working memory (run table, sorted copy of the particles, supercell histogram and starts, position
+// records, permutation) lives in `scratch`, one file-scope device array per GPU that
 // stays allocated until the process ends. Host code never passes the array's name to a kernel: the
 // name is a host-side stand-in, not a device address. The device address is taken once per device
 // with hipGetSymbolAddress and kept in `g_scratch`. Every call on a GPU shares its array, so calls
-// that overlap on one GPU (different streams or threads) race; each call clears what must start at
-// zero (the supercell histogram) with a fill kernel.
+// that overlap on one GPU (different streams or threads) race; each call's first kernel clears what must
+// start at zero (the supercell histogram) and sets the rest up.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
